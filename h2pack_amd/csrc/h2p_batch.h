@@ -130,12 +130,7 @@ __global__ void __launch_bounds__(256) k_leaf_final2_b(const BatchItem *__restri
 // Co-scheduled multi-RHS products: one launch per matmul phase serves every
 // request of the batch, each with its own panels.
 struct MMCtx {
-    const MMSrc *srcs;
-    const double *shifts;
-    const double *U, *UT, *BD, *coord;
-    long long CT;
-    KParam kp;
-    MMPanels P;
+    MMArgs A;
     const int *fwd;
     int N, nv;           // points x kd, vectors of this chunk
     const double *X;     // caller panels
@@ -144,31 +139,37 @@ struct MMCtx {
     int row_major, v0;
 };
 
-template <int KID, int KD, class G>
-__global__ void __launch_bounds__(256) k_mm_b(const BatchItem *__restrict__ items, int n,
-                                              const MMCtx *__restrict__ reqs) {
+template <int NVT>
+__global__ void __launch_bounds__(256) k_mmd_b(const BatchItem *__restrict__ items, int n,
+                                               const MMCtx *__restrict__ reqs) {
     const int it = find_item(items, n, blockIdx.x);
     const MMCtx &c = reqs[items[it].req];
-    const MMTask t = ((const MMTask *)items[it].tasks)[blockIdx.x - items[it].begin];
-    mm_body<KID, KD, G>(t, c.srcs, c.U, c.UT, c.BD, c.coord, c.CT, c.kp, c.shifts, c.P);
+    mmd_body<NVT, true>(((const MMTask *)items[it].tasks)[blockIdx.x - items[it].begin], c.A);
+}
+
+template <int KID, int NVT>
+__global__ void __launch_bounds__(256) k_mmj_b(const BatchItem *__restrict__ items, int n,
+                                               const MMCtx *__restrict__ reqs) {
+    const int it = find_item(items, n, blockIdx.x);
+    const MMCtx &c = reqs[items[it].req];
+    mmj_body<KID, NVT, true>(((const MMTask *)items[it].tasks)[blockIdx.x - items[it].begin], c.A);
 }
 
 // The FP32-mixed product phases (coupling, and the B/D part of the leaves)
-// of FP32-mixed handles; BD is then the FP32 block store (AOT).
-template <int KID, class G>
+// of FP32-mixed handles.
+template <int KID, int NVT>
 __global__ void __launch_bounds__(256) k_mm32_b(const BatchItem *__restrict__ items, int n,
                                                 const MMCtx *__restrict__ reqs) {
     const int it = find_item(items, n, blockIdx.x);
     const MMCtx &c = reqs[items[it].req];
-    const MMTask t = ((const MMTask *)items[it].tasks)[blockIdx.x - items[it].begin];
-    mm32_body<KID, G>(t, c.srcs, (const float *)c.BD, c.coord, c.CT, (float)c.kp.p0, c.shifts, c.P);
+    mm32_body<KID, NVT, true>(((const MMTask *)items[it].tasks)[blockIdx.x - items[it].begin], c.A);
 }
 
 __global__ void __launch_bounds__(256) k_mm_gather_b(const BatchItem *__restrict__ items, int n,
                                                      const MMCtx *__restrict__ reqs) {
     const int it = find_item(items, n, blockIdx.x);
     const MMCtx &c = reqs[items[it].req];
-    const int nvp = c.P.nvp;
+    const int nvp = c.A.P.nvp;
     const long long e = (long long)(blockIdx.x - items[it].begin) * 256 + threadIdx.x;
     if (e >= (long long)c.N * nvp) return;
     const int i = (int)(e / nvp), col = (int)(e - (long long)i * nvp);
@@ -177,7 +178,7 @@ __global__ void __launch_bounds__(256) k_mm_gather_b(const BatchItem *__restrict
         const long long src = c.fwd[i];
         v = c.row_major ? c.X[src * c.ldx + c.v0 + col] : c.X[(long long)(c.v0 + col) * c.ldx + src];
     }
-    c.P.p[MM_PX][e] = v;
+    c.A.P.p[MM_PX][e] = v;
 }
 
 __global__ void __launch_bounds__(256) k_mm_scatter_b(const BatchItem *__restrict__ items, int n,
@@ -188,7 +189,7 @@ __global__ void __launch_bounds__(256) k_mm_scatter_b(const BatchItem *__restric
     if (e >= (long long)c.N * c.nv) return;
     const int i = (int)(e / c.nv), col = (int)(e - (long long)i * c.nv);
     const long long dstr = c.fwd[i];
-    const double v = c.P.p[MM_PY][(long long)i * c.P.nvp + col];
+    const double v = c.A.P.p[MM_PY][(long long)i * c.A.P.nvp + col];
     if (c.row_major) c.Y[dstr * c.ldy + c.v0 + col] = v;
     else c.Y[(long long)(c.v0 + col) * c.ldy + dstr] = v;
 }

@@ -88,10 +88,18 @@ H2P_HD inline double exp2_neg128(double x, const double *tab) {
     return __builtin_ldexp(__builtin_fma(T * u, p, T), m);
 }
 
-// The same for any x >= 0 (or +inf): x is clamped to 128 * 1100 first,
-// where the result is already 0.
+// The same for any x >= 0 (or +inf): x is clamped to about 128 * 1100 first,
+// where the result is already 0.  The clamp is one integer minimum on the
+// upper word (0x41013000 is that of 128 * 1100): non-negative doubles order as
+// their upper words do and the lower word left behind stays below the next
+// one, while fmin costs a second FP64 operation that quiets its argument.
 H2P_HD inline double exp2_neg128_clamped(double x, const double *tab) {
-    return exp2_neg128(__builtin_fmin(x, 128.0 * 1100.0), tab);
+    uint64_t b;
+    __builtin_memcpy(&b, &x, sizeof b);
+    const int32_t hi = (int32_t)(b >> 32), cl = 0x41013000;
+    b = ((uint64_t)(uint32_t)(hi < cl ? hi : cl) << 32) | (uint32_t)b;
+    __builtin_memcpy(&x, &b, sizeof b);
+    return exp2_neg128(x, tab);
 }
 
 }  // namespace h2p

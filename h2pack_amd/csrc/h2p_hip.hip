@@ -107,7 +107,7 @@ struct h2p_hip_handle {
     double *d_mm_x = nullptr, *d_mm_y = nullptr;  // staging of the host-pointer calls
     size_t mm_cap = 0;
     // matmul (pull-form MFMA tasks, built at upload)
-    MMTask *d_mmt = nullptr;
+    MMTask *d_mmt = nullptr, *d_mmt_l = nullptr;   // the tasks in both orders (task_orders)
     MMSrc *d_mms = nullptr;
     std::vector<Level> mm_fwd_levels, mm_bwd_levels;
     std::vector<BlkTask> h_blk;   // host copies, for the autotuner's histograms
@@ -121,7 +121,7 @@ struct h2p_hip_handle {
     Level mm_leaf32{0, 0};
     double *d_panels = nullptr;   // PX | Y0 | Y1 | PY, panel_nvp wide
     int panel_nvp = 0;
-    int mm_var[4][3] = {};        // tile variant per matmul phase and panel width class
+    int mm_var[4][3] = {};        // variant (task order) per matmul phase and panel width class
     int mv_var = 0;               // variant of the matvec block launch (0 default, 1 other occupancy)
     // FP64 Gaussian / Matern JIT: the point extent can push the exponential's
     // argument past the unclamped range, so the launches use KGW / KMW
@@ -199,7 +199,7 @@ static void free_handle(h2p_hip_handle *h) {
     if (!h) return;
     void *ptrs[] = {h->d_coord, h->d_U, h->d_UT, h->d_blob, h->d_xin, h->d_y1, h->d_arena,
                     h->d_fwd, h->d_blk, h->d_fwdt, h->d_bwdt, h->d_red, h->d_leaf,
-                    h->d_contrib, h->d_mm_x, h->d_mm_y, h->d_yp, h->d_yt, h->d_mmt, h->d_mms, h->d_panels,
+                    h->d_contrib, h->d_mm_x, h->d_mm_y, h->d_yp, h->d_yt, h->d_mmt, h->d_mmt_l, h->d_mms, h->d_panels,
                     h->d_cg, h->d_shift, h->d_per};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -556,78 +556,62 @@ static int run_matvec(h2p_hip_handle *h, const double *d_x, double *d_y, hipStre
     return 0;
 }
 
-// matmul launches: kernel dimension and id, panel width class (NV = 16, 32
-// or 64 columns) and tile variant (chosen by h2p_hip_autotune)
+// matmul panel width classes of the variants (16, 32 or 64 columns)
 static int nv_class(int nvp) { return nvp <= 16 ? 0 : nvp <= 32 ? 1 : 2; }
 
-template <int KID, int KD, int NV, int V>
-static void launch_mm_v(const h2p_hip_handle *h, const Level &L, const MMPanels &P, hipStream_t s) {
+static MMArgs mm_args(const h2p_hip_handle *h, const MMPanels &P) {
+    MMArgs A{};
+    A.srcs = h->d_mms;
+    A.U = h->d_U;
+    A.UT = h->d_UT;
     // dense B/D sources: the stored blocks, or in periodic mode the root's block
-    const double *bd = h->periodic ? h->d_per : (const double *)h->d_blob;
-    hipLaunchKernelGGL((k_mm<KID, KD, MMVar<KD, NV, V>>), dim3(L.n), dim3(256), 0, s, h->d_mmt + L.off, h->d_mms,
-                       h->d_U, h->d_UT, bd, h->d_coord, h->CT, h->kp, h->d_shift, P);
+    A.BD = h->periodic ? (const void *)h->d_per : h->d_blob;
+    A.cx = h->d_coord;
+    A.cstride = h->CT;
+    A.shifts = h->d_shift;
+    A.scale = kscale(h->kid, h->kp.p0, true);
+    A.kp = h->kp;
+    A.P = P;
+    return A;
 }
 
-template <int KID, int KD, int NV>
-static void launch_mm_nv(const h2p_hip_handle *h, const Level &L, const MMPanels &P, hipStream_t s, int v) {
-    switch (v) {
-        case 1: launch_mm_v<KID, KD, NV, 1>(h, L, P, s); break;
-        case 2: launch_mm_v<KID, KD, NV, 2>(h, L, P, s); break;
-        case 3: launch_mm_v<KID, KD, NV, 3>(h, L, P, s); break;
-        default: launch_mm_v<KID, KD, NV, 0>(h, L, P, s); break;
+// What a phase's tasks hold: dense sources only, evaluated ones too, or the
+// FP32-mixed block products.
+enum { MMK_DENSE = 0, MMK_JIT = 1, MMK_F32 = 2 };
+
+template <int NVT>
+static void launch_mm(const h2p_hip_handle *h, int kind, const MMTask *tasks, int n, const MMArgs &A, hipStream_t s) {
+    const dim3 g(n), b(256);
+    if (kind == MMK_DENSE) {
+        hipLaunchKernelGGL((k_mmd<NVT>), g, b, 0, s, tasks, A);
+    } else if (kind == MMK_JIT) {
+        switch (h->kid) {
+            case KC: hipLaunchKernelGGL((k_mmj<KC, NVT>), g, b, 0, s, tasks, A); break;
+            case KG: hipLaunchKernelGGL((k_mmj<KGW, NVT>), g, b, 0, s, tasks, A); break;
+            case KM: hipLaunchKernelGGL((k_mmj<KMW, NVT>), g, b, 0, s, tasks, A); break;
+            default: hipLaunchKernelGGL((k_mmj<KR, NVT>), g, b, 0, s, tasks, A); break;
+        }
+    } else if (h->mode == H2P_HIP_AOT) {
+        hipLaunchKernelGGL((k_mm32<-1, NVT>), g, b, 0, s, tasks, A);
+    } else {
+        switch (h->kid) {
+            case KC: hipLaunchKernelGGL((k_mm32<KC, NVT>), g, b, 0, s, tasks, A); break;
+            case KG: hipLaunchKernelGGL((k_mm32<KG, NVT>), g, b, 0, s, tasks, A); break;
+            default: hipLaunchKernelGGL((k_mm32<KM, NVT>), g, b, 0, s, tasks, A); break;
+        }
     }
 }
 
-template <int KID, int KD>
-static void launch_mm(const h2p_hip_handle *h, const Level &L, const MMPanels &P, hipStream_t s, int v) {
-    switch (nv_class(P.nvp)) {
-        case 0: launch_mm_nv<KID, KD, 16>(h, L, P, s, v); break;
-        case 1: launch_mm_nv<KID, KD, 32>(h, L, P, s, v); break;
-        default: launch_mm_nv<KID, KD, 64>(h, L, P, s, v); break;
-    }
-}
-
-static void dispatch_mm(const h2p_hip_handle *h, const Level &L, const MMPanels &P, hipStream_t s, int v) {
+// Variant v of one launch: bit 0 picks the task order (the other bit is free).
+static void dispatch_mm(const h2p_hip_handle *h, int kind, const Level &L, const MMPanels &P, hipStream_t s, int v) {
     if (L.n <= 0) return;
-    switch (h->kid) {
-        case KC: launch_mm<KC, 1>(h, L, P, s, v); break;
-        case KG: launch_mm<KG, 1>(h, L, P, s, v); break;
-        case KM: launch_mm<KM, 1>(h, L, P, s, v); break;
-        default: launch_mm<KR, 3>(h, L, P, s, v); break;
-    }
-}
-
-template <int KID, int NV, int V>
-static void launch_mm32_v(const h2p_hip_handle *h, const Level &L, const MMPanels &P, hipStream_t s) {
-    hipLaunchKernelGGL((k_mm32<KID, MMVar<1, NV, V>>), dim3(L.n), dim3(256), 0, s, h->d_mmt + L.off, h->d_mms,
-                       (const float *)h->d_blob, h->d_coord, h->CT, (float)h->kp.p0, h->d_shift, P);
-}
-
-template <int KID, int NV>
-static void launch_mm32_nv(const h2p_hip_handle *h, const Level &L, const MMPanels &P, hipStream_t s, int v) {
-    switch (v) {
-        case 1: launch_mm32_v<KID, NV, 1>(h, L, P, s); break;
-        case 2: launch_mm32_v<KID, NV, 2>(h, L, P, s); break;
-        case 3: launch_mm32_v<KID, NV, 3>(h, L, P, s); break;
-        default: launch_mm32_v<KID, NV, 0>(h, L, P, s); break;
-    }
-}
-
-template <int KID>
-static void launch_mm32(const h2p_hip_handle *h, const Level &L, const MMPanels &P, hipStream_t s, int v) {
-    switch (nv_class(P.nvp)) {
-        case 0: launch_mm32_nv<KID, 16>(h, L, P, s, v); break;
-        case 1: launch_mm32_nv<KID, 32>(h, L, P, s, v); break;
-        default: launch_mm32_nv<KID, 64>(h, L, P, s, v); break;
-    }
-}
-
-static void dispatch_mm32(const h2p_hip_handle *h, const Level &L, const MMPanels &P, hipStream_t s, int v) {
-    if (L.n <= 0) return;
-    switch (h->kid) {
-        case KC: launch_mm32<KC>(h, L, P, s, v); break;
-        case KG: launch_mm32<KG>(h, L, P, s, v); break;
-        default: launch_mm32<KM>(h, L, P, s, v); break;
+    const MMArgs A = mm_args(h, P);
+    const MMTask *tasks = ((v & 1) ? h->d_mmt_l : h->d_mmt) + L.off;
+    switch (P.nvp >> 4) {
+        case 1: launch_mm<1>(h, kind, tasks, L.n, A, s); break;
+        case 2: launch_mm<2>(h, kind, tasks, L.n, A, s); break;
+        case 3: launch_mm<3>(h, kind, tasks, L.n, A, s); break;
+        default: launch_mm<4>(h, kind, tasks, L.n, A, s); break;
     }
 }
 
@@ -651,8 +635,9 @@ static std::vector<Level> mm_phase_levels32(const h2p_hip_handle *h, int ph) {
 }
 
 static void launch_mm_phase(const h2p_hip_handle *h, int ph, const MMPanels &P, hipStream_t s, int v) {
-    for (const Level &L : mm_phase_levels(h, ph)) dispatch_mm(h, L, P, s, v);
-    for (const Level &L : mm_phase_levels32(h, ph)) dispatch_mm32(h, L, P, s, v);
+    const int kind = h->mode == H2P_HIP_JIT && !h->mm_f32 && (ph == MMP_INTMD || ph == MMP_LEAF) ? MMK_JIT : MMK_DENSE;
+    for (const Level &L : mm_phase_levels(h, ph)) dispatch_mm(h, kind, L, P, s, v);
+    for (const Level &L : mm_phase_levels32(h, ph)) dispatch_mm(h, MMK_F32, L, P, s, v);
 }
 
 static void drop_mm_graphs(h2p_hip_handle *h) {
@@ -1143,7 +1128,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
     }
     h->n_leaf = (int)leaf.size();
     // ---- matmul tasks (pull form, one task per destination)
-    std::vector<MMTask> mmt;
+    std::vector<MMTask> mmt, mmt_l;
     std::vector<MMSrc> mms;
     const bool jit = mode == H2P_HIP_JIT;
     const bool mm_f32 = prec == H2P_HIP_FP32MIX && krnl->id != KR && !per;
@@ -1164,14 +1149,14 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             a.lda = b.lda = bc;
             // entry of n0: op = B
             a.trans = 0; a.K = bc;
-            a.c0 = set_start(n0, p0); a.c1 = set_start(n1, p1);
+            a.c1 = set_start(n1, p1);
             a.x_space = p1 ? MM_PX : MM_Y0; a.x_off = p1 ? g->mat_cluster[2 * n1] : soff[n1];
             a.shift = adm_shift[i];
             (p0 ? leaf_src[n0] : y1_src[n0]).push_back(a);
             if (per) continue;   // one-sided pairs
             // entry of n1: op = B^T
             b.trans = 1; b.K = br;
-            b.c0 = set_start(n1, p1); b.c1 = set_start(n0, p0);
+            b.c1 = set_start(n0, p0);
             b.x_space = p0 ? MM_PX : MM_Y0; b.x_off = p0 ? g->mat_cluster[2 * n0] : soff[n0];
             (p1 ? leaf_src[n1] : y1_src[n1]).push_back(b);
         }
@@ -1186,43 +1171,83 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             a.a_off = (long long)(btot + g->D_ptr[i]);
             a.lda = dc;
             a.trans = 0; a.K = dc;
-            a.c0 = g->pt_cluster[2 * n0]; a.c1 = g->pt_cluster[2 * n1];
+            a.c1 = g->pt_cluster[2 * n1];
             a.x_space = MM_PX; a.x_off = g->mat_cluster[2 * n1];
             if (i >= nlf) a.shift = inadm_shift[i - nlf];
             leaf_src[n0].push_back(a);
             if (i >= nlf && !per) {
                 MMSrc b = a;
                 b.trans = 1; b.K = dr;
-                b.c0 = g->pt_cluster[2 * n1]; b.c1 = g->pt_cluster[2 * n0];
+                b.c1 = g->pt_cluster[2 * n0];
                 b.x_off = g->mat_cluster[2 * n0];
                 leaf_src[n1].push_back(b);
             }
         }
-        // a destination of M rows becomes tasks of at most MM_PIECE rows (a
-        // multiple of every variant's row chunk, and of 3 for whole points),
-        // each with its sources restricted to its rows: more workgroups for
-        // the few large destinations of the upper levels, the same MFMA
-        // sequence per output element, one writer per row
-        const int MM_PIECE = kd == 3 ? 96 : 128;
-        auto add_task = [&](int space, int off, int M, int accum, const std::vector<MMSrc> &src) {
-            for (int m0 = 0; m0 < M || (M == 0 && m0 == 0); m0 += MM_PIECE) {
+        // A destination of M rows becomes tasks of at most `piece` rows that
+        // share its source list (dense sources first), with one writer per
+        // row.  Tasks with evaluated 3x3 blocks hold 16 points, the others
+        // 32 rows.
+        auto add_task = [&](int space, int off, int M, int accum, const std::vector<MMSrc> &src, int c0, int piece) {
+            const int sbeg = (int)mms.size();
+            for (const MMSrc &x : src)
+                if (x.kind != MM_A_JIT && x.K > 0) mms.push_back(x);
+            const int smid = (int)mms.size();
+            for (const MMSrc &x : src)
+                if (x.kind == MM_A_JIT && x.K > 0) mms.push_back(x);
+            const int send = (int)mms.size();
+            for (int m0 = 0; m0 < M; m0 += piece) {
                 MMTask t{};
-                t.dst_space = space; t.dst_off = off + m0; t.M = std::min(MM_PIECE, M - m0); t.accumulate = accum;
-                t.sbeg = (int)mms.size();
-                for (MMSrc x : src) {
-                    if (x.kind == MM_A_JIT) x.c0 += m0 / kd;
-                    else x.a_off += x.trans ? (long long)m0 : (long long)m0 * x.lda;
-                    mms.push_back(x);
-                }
-                t.send = (int)mms.size();
+                t.dst_space = space; t.dst_off = off + m0; t.M = std::min(piece, M - m0); t.accumulate = accum;
+                t.sbeg = sbeg; t.smid = smid; t.send = send;
+                t.m0 = m0;
+                t.c0 = c0 + m0 / kd;
                 mmt.push_back(t);
-                if (M == 0) break;
             }
         };
-        auto work = [&](const MMTask &t) {
-            long long wsum = 0;
-            for (int k = t.sbeg; k < t.send; k++) wsum += (long long)t.M * mms[k].K;
-            return wsum;
+        const int jpiece = jit && kd == 3 ? H2P_MM_PIECE3 : H2P_MM_PIECE;   // coupling and leaf tasks
+        // Two orders of a phase's tasks.  mmt (variant 0): destinations by
+        // the work of all their tasks, eight at a time, their tasks dealt in
+        // turn, so that the tasks of one destination, which read the same
+        // operand rows, fall on one XCD and its L2 (workgroups go round the
+        // eight XCDs).  mmt_l (variant 1): single tasks, longest first (rows
+        // x inner entries).  Measured, grouped against longest first, ms per
+        // product: RPY N = 20k x32 3.10 / 3.62, Coulomb N = 80k x20 2.28 /
+        // 2.52, Gaussian N = 17k AOT x64 1.00 / 1.14; eight contiguous
+        // spatial ranges of destinations, one per XCD, gave 3.27 / 2.47 / 1.11.
+        auto task_orders = [&](const Level &L) {
+            std::vector<MMTask> in(mmt.begin() + L.off, mmt.begin() + L.off + L.n), v;
+            std::vector<std::pair<long long, int>> key(L.n), dst;   // (-work, first task); dst: per destination
+            std::vector<int> dn;
+            for (int i = 0; i < L.n;) {
+                long long ksum = 0, tot = 0;
+                for (int k = in[i].sbeg; k < in[i].send; k++) ksum += mms[k].K;
+                int j = i;
+                do {
+                    key[j] = {-(long long)in[j].M * ksum, j};
+                    tot += key[j].first;
+                    j++;
+                } while (j < L.n && in[j].m0 > 0);
+                dst.push_back({tot, (int)dn.size()});
+                dn.push_back(i);
+                i = j;
+            }
+            dn.push_back(L.n);
+            std::sort(key.begin(), key.end());
+            mmt_l.resize(mmt.size());
+            for (int i = 0; i < L.n; i++) mmt_l[L.off + i] = in[key[i].second];
+            std::sort(dst.begin(), dst.end());
+            for (size_t d = 0; d < dst.size(); d += 8)
+                for (int j = 0, more = 1; more; j++) {
+                    more = 0;
+                    for (size_t q = d; q < std::min(dst.size(), d + 8); q++) {
+                        const int b = dn[dst[q].second], e = dn[dst[q].second + 1];
+                        if (b + j < e) {
+                            v.push_back(in[b + j]);
+                            more = 1;
+                        }
+                    }
+                }
+            std::copy(v.begin(), v.end(), mmt.begin() + L.off);
         };
         // upward sweep, level by level
         for (int lv = g->max_level; lv >= g->min_adm_level; lv--) {
@@ -1234,9 +1259,10 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
                 a.kind = MM_A_UT; a.a_off = uoff[n]; a.lda = g->U_nrow[n]; a.trans = 0; a.K = g->U_nrow[n];
                 if (g->n_child[n] == 0) { a.x_space = MM_PX; a.x_off = g->mat_cluster[2 * n]; }
                 else { a.x_space = MM_Y0; a.x_off = soff[g->children[(size_t)n * mc]]; }
-                add_task(MM_Y0, soff[n], g->U_ncol[n], 0, std::vector<MMSrc>{a});
+                add_task(MM_Y0, soff[n], g->U_ncol[n], 0, std::vector<MMSrc>{a}, 0, H2P_MM_PIECE);
             }
             L.n = (int)mmt.size() - L.off;
+            task_orders(L);
             if (L.n > 0) h->mm_fwd_levels.push_back(L);
         }
         // periodic: the root's block, a dense source on its own skeleton
@@ -1251,9 +1277,10 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
         {
             Level L{(int)mmt.size(), 0};
             for (int n = 0; n < nn; n++)
-                if (g->U_ncol[n] > 0) add_task(MM_Y1, soff[n], g->U_ncol[n], 0, y1_src[n]);
+                if (g->U_ncol[n] > 0)
+                    add_task(MM_Y1, soff[n], g->U_ncol[n], 0, y1_src[n], set_start(n, false), jpiece);
             L.n = (int)mmt.size() - L.off;
-            std::stable_sort(mmt.begin() + L.off, mmt.end(), [&](const MMTask &x, const MMTask &y) { return work(x) > work(y); });
+            task_orders(L);
             h->mm_intmd = L;
         }
         // downward sweep, level by level
@@ -1265,9 +1292,10 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
                 MMSrc a{};
                 a.kind = MM_A_U; a.a_off = uoff[n]; a.lda = g->U_ncol[n]; a.trans = 0; a.K = g->U_ncol[n];
                 a.x_space = MM_Y1; a.x_off = soff[n];
-                add_task(MM_Y1, soff[g->children[(size_t)n * mc]], g->U_nrow[n], 1, std::vector<MMSrc>{a});
+                add_task(MM_Y1, soff[g->children[(size_t)n * mc]], g->U_nrow[n], 1, std::vector<MMSrc>{a}, 0, H2P_MM_PIECE);
             }
             L.n = (int)mmt.size() - L.off;
+            task_orders(L);
             if (L.n > 0) h->mm_bwd_levels.push_back(L);
         }
         // leaf outputs; FP32-mixed handles split them into the U part (FP64
@@ -1285,19 +1313,20 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
                 }
                 if (!mm_f32)
                     for (const MMSrc &x : leaf_src[n]) src.push_back(x);
-                add_task(MM_PY, g->mat_cluster[2 * n], npt(n) * kd, 0, src);
+                add_task(MM_PY, g->mat_cluster[2 * n], npt(n) * kd, 0, src, set_start(n, true), jpiece);
             }
             L.n = (int)mmt.size() - L.off;
-            std::stable_sort(mmt.begin() + L.off, mmt.end(), [&](const MMTask &x, const MMTask &y) { return work(x) > work(y); });
+            task_orders(L);
             h->mm_leaf = L;
             if (mm_f32) {
                 Level L32{(int)mmt.size(), 0};
                 for (int i = 0; i < nlf; i++) {
                     int n = g->leaf_nodes[i];
-                    if (!leaf_src[n].empty()) add_task(MM_PY, g->mat_cluster[2 * n], npt(n) * kd, 1, leaf_src[n]);
+                    if (!leaf_src[n].empty())
+                        add_task(MM_PY, g->mat_cluster[2 * n], npt(n) * kd, 1, leaf_src[n], set_start(n, true), jpiece);
                 }
                 L32.n = (int)mmt.size() - L32.off;
-                std::stable_sort(mmt.begin() + L32.off, mmt.end(), [&](const MMTask &x, const MMTask &y) { return work(x) > work(y); });
+                task_orders(L32);
                 h->mm_leaf32 = L32;
             }
         }
@@ -1345,21 +1374,26 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             if (fwdidx_ok(g->fwd_pmt_idx[i], N) == false) return bail(fail(H2P_HIP_EINVAL, "fwd_pmt_idx out of range"));
         const long long rows_of[4] = {N, S, S, N};
         for (const MMTask &t : mmt) {
-            bool ok = t.dst_space >= 0 && t.dst_space < 4 && in(t.dst_off, t.M, rows_of[t.dst_space]) &&
-                      t.sbeg >= 0 && t.send >= t.sbeg && t.send <= (int)mms.size();
+            const int piece = t.smid < t.send && kd == 3 ? H2P_MM_PIECE3 : std::max(H2P_MM_PIECE, jit && kd == 3 ? H2P_MM_PIECE3 : 0);
+            bool ok = t.dst_space >= 0 && t.dst_space < 4 && t.M > 0 && t.M <= piece && t.m0 >= 0 &&
+                      in(t.dst_off, t.M, rows_of[t.dst_space]) && t.sbeg >= 0 && t.smid >= t.sbeg &&
+                      t.send >= t.smid && t.send <= (int)mms.size();
+            if (ok && t.smid < t.send) ok = t.M % kd == 0 && in(t.c0, t.M / kd, CT);
             for (int k = t.sbeg; ok && k < t.send; k++) {
                 const MMSrc &x = mms[k];
-                ok = x.x_space >= 0 && x.x_space < 4 && in(x.x_off, x.K, rows_of[x.x_space]) && x.K >= 0;
+                ok = x.x_space >= 0 && x.x_space < 4 && x.K > 0 && in(x.x_off, x.K, rows_of[x.x_space]);
                 if (!ok) break;
-                if (x.kind == MM_A_JIT) {
-                    ok = (t.M % kd == 0) && (x.K % kd == 0) && in(x.c0, t.M / kd, CT) && in(x.c1, x.K / kd, CT) &&
-                         x.shift >= 0 && x.shift < (int)(shtab.size() / 3);
+                if (k >= t.smid) {
+                    ok = x.kind == MM_A_JIT && x.K % kd == 0 && in(x.c1, x.K / kd, CT) && x.shift >= 0 &&
+                         x.shift < (int)(shtab.size() / 3);
                 } else {
+                    // rows m0 .. m0 + M - 1 of op(A)
                     const long long per_cap = (long long)g->U_ncol[root] * g->U_ncol[root];
                     const long long cap = (x.kind == MM_A_BD) ? (per ? per_cap : BLOB) : utot;
-                    const long long rows = x.trans ? x.K : t.M, cols = x.trans ? t.M : x.K;
+                    const long long m1 = (long long)t.m0 + t.M;
+                    const long long rows = x.trans ? x.K : m1, cols = x.trans ? m1 : x.K;
                     ok = (x.kind == MM_A_U || x.kind == MM_A_UT || x.kind == MM_A_BD) && x.lda >= cols &&
-                         (rows == 0 || in(x.a_off, (rows - 1) * (long long)x.lda + cols, cap));
+                         in(x.a_off, (rows - 1) * (long long)x.lda + cols, cap);
                 }
             }
             if (!ok) return bail(fail(H2P_HIP_EINVAL, "matmul task out of range"));
@@ -1437,7 +1471,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             return sizeof(typename std::decay_t<decltype(v)>::value_type) * std::max<size_t>(v.size(), 1);
         };
         size_t b = vb(cu) + vb(Ub) + vb(UTb) + sizeof(int) * std::max<size_t>(N, 1) + vb(blk) + vb(fwdt) +
-                   vb(bwdt) + vb(red) + vb(leaf) + vb(contrib) + vb(mmt) + vb(mms) + vb(shtab) +
+                   vb(bwdt) + vb(red) + vb(leaf) + vb(contrib) + 2 * vb(mmt) + vb(mms) + vb(shtab) +
                    (per ? sizeof(double) * per_elems : 0);
         b += sizeof(double) * (std::max<size_t>((size_t)N + S, 1) + 2 * std::max<size_t>(S, 1) +
                                std::max<size_t>((size_t)arena, 1));
@@ -1463,6 +1497,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
     if ((rc = dev_upload(&h->d_leaf, leaf, acct))) return bail(rc);
     if ((rc = dev_upload(&h->d_contrib, contrib, acct))) return bail(rc);
     if ((rc = dev_upload(&h->d_mmt, mmt, acct))) return bail(rc);
+    if ((rc = dev_upload(&h->d_mmt_l, mmt_l, acct))) return bail(rc);
     if ((rc = dev_upload(&h->d_mms, mms, acct))) return bail(rc);
     if ((rc = dev_upload(&h->d_shift, shtab, acct))) return bail(rc);
     if (per) {
@@ -1965,7 +2000,7 @@ int h2p_hip_autotune(h2p_hip_handle *h, int n_vec, double *t_default_ms, double 
         for (const Level &L : mm_phase_levels32(h, ph)) empty = empty && L.n <= 0;
         if (empty) continue;
         const std::string sig = tune_signature(h, ph, cls, h->h_mmt, h->h_mms);
-        double t[H2P_MM_NVARIANT];
+        double t[2];
         int best = 0;
         {
             std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -1977,7 +2012,7 @@ int h2p_hip_autotune(h2p_hip_handle *h, int n_vec, double *t_default_ms, double 
             }
         }
         const int reps = 3;
-        for (int v = 0; v < H2P_MM_NVARIANT && !err; v++) {
+        for (int v = 0; v < 2 && !err; v++) {   // the two task orders
             launch_mm_phase(h, ph, P, s, v);   // warm-up
             if (hipEventRecord(e0, s) != hipSuccess) { err = 1; break; }
             for (int r = 0; r < reps; r++) launch_mm_phase(h, ph, P, s, v);
@@ -2319,6 +2354,30 @@ static void launch_matvec_b(const MVPlan &P, const char *dbase, hipStream_t s) {
     launch_items(k_leaf_final2_b, P.leaf, dbase, reqs, s);
 }
 
+// A batched product phase on panels of at most 16 NVT columns.
+template <int NVT>
+static void launch_mm_b(int kind, int kid, const BatchItem *it, const BLaunch &b, const MMCtx *reqs, hipStream_t s) {
+    const dim3 g(b.grid), blk(256);
+    const int n = b.n_items;
+    if (kind == MMK_DENSE) {
+        hipLaunchKernelGGL((k_mmd_b<NVT>), g, blk, 0, s, it, n, reqs);
+    } else if (kind == MMK_JIT) {
+        switch (kid) {
+            case KC: hipLaunchKernelGGL((k_mmj_b<KC, NVT>), g, blk, 0, s, it, n, reqs); break;
+            case KG: hipLaunchKernelGGL((k_mmj_b<KGW, NVT>), g, blk, 0, s, it, n, reqs); break;
+            case KM: hipLaunchKernelGGL((k_mmj_b<KMW, NVT>), g, blk, 0, s, it, n, reqs); break;
+            default: hipLaunchKernelGGL((k_mmj_b<KR, NVT>), g, blk, 0, s, it, n, reqs); break;
+        }
+    } else {
+        switch (kid) {
+            case KC: hipLaunchKernelGGL((k_mm32_b<KC, NVT>), g, blk, 0, s, it, n, reqs); break;
+            case KG: hipLaunchKernelGGL((k_mm32_b<KG, NVT>), g, blk, 0, s, it, n, reqs); break;
+            case KM: hipLaunchKernelGGL((k_mm32_b<KM, NVT>), g, blk, 0, s, it, n, reqs); break;
+            default: hipLaunchKernelGGL((k_mm32_b<-1, NVT>), g, blk, 0, s, it, n, reqs); break;
+        }
+    }
+}
+
 struct CGPlan {
     size_t cgs_off = 0, first_off = 0;
     int n = 0, grid = 0;
@@ -2496,15 +2555,7 @@ int h2p_hip_matmul_batch(h2p_hip_batch *B, int n, h2p_hip_handle *const *hs, int
             h2p_hip_handle *h = hs[i];
             MMCtx c{};
             c.nv = std::min(H2P_MM_MAXNVP, n_vec[i] - v0);
-            c.srcs = h->d_mms;
-            c.shifts = h->d_shift;
-            c.U = h->d_U;
-            c.UT = h->d_UT;
-            c.BD = (const double *)h->d_blob;
-            c.coord = h->d_coord;
-            c.CT = h->CT;
-            c.kp = h->kp;
-            c.P = panels_of(h, (c.nv + 15) & ~15, h->d_panels);
+            c.A = mm_args(h, panels_of(h, (c.nv + 15) & ~15, h->d_panels));
             c.fwd = h->d_fwd;
             c.N = h->N;
             c.X = d_X[i];
@@ -2522,41 +2573,48 @@ int h2p_hip_matmul_batch(h2p_hip_batch *B, int n, h2p_hip_handle *const *hs, int
         ItemList g, sc;
         size_t max_fwd = 0, max_bwd = 0;
         for (int i = 0; i < m; i++) {
-            const long long ne = (long long)act[i]->N * ctx[i].P.nvp, no = (long long)act[i]->N * ctx[i].nv;
+            const long long ne = (long long)act[i]->N * ctx[i].A.P.nvp, no = (long long)act[i]->N * ctx[i].nv;
             g.add(i, nullptr, (int)((ne + 255) / 256));
             sc.add(i, nullptr, (int)((no + 255) / 256));
             max_fwd = std::max(max_fwd, act[i]->mm_fwd_levels.size());
             max_bwd = std::max(max_bwd, act[i]->mm_bwd_levels.size());
         }
         const BLaunch lg = finish(tb, g), ls = finish(tb, sc);
-        // product phases, grouped by kernel id: (level list, launch)
-        // (FP32-mixed handles run their coupling phase and the B/D part of
-        // their leaf outputs in the FP32 kernel: grouped apart)
-        struct MMLaunch { BLaunch b; int kid; bool f32; };
+        // product phases, grouped by the kernel that runs them: dense tasks
+        // of every handle together, evaluated ones by kernel id, FP32-mixed
+        // ones by kernel id and mode
+        struct MMLaunch { BLaunch b; int kind, kid; };
         std::vector<MMLaunch> phases;
-        auto add_phase = [&](auto level_of, bool coupling) {
+        auto kernel_of = [](const h2p_hip_handle *h, bool blocks, bool f32) {
+            if (f32) return std::make_pair((int)MMK_F32, h->mode == H2P_HIP_AOT ? -1 : h->kid);
+            if (blocks && h->mode == H2P_HIP_JIT && !h->mm_f32) return std::make_pair((int)MMK_JIT, h->kid);
+            return std::make_pair((int)MMK_DENSE, 0);
+        };
+        // blocks: a phase with B/D sources (coupling, leaves); split32: the
+        // phase's FP32-mixed part
+        auto add_phase = [&](auto level_of, bool blocks, bool split32) {
             std::vector<int> used(m, 0);
             for (int i = 0; i < m; i++) {
                 if (used[i]) continue;
-                const bool f32 = coupling && act[i]->mm_f32;
+                const auto key = kernel_of(act[i], blocks, split32 && act[i]->mm_f32);
                 ItemList L;
                 for (int j = i; j < m; j++) {
-                    if (used[j] || act[j]->kid != act[i]->kid || (coupling && act[j]->mm_f32) != f32) continue;
+                    if (used[j] || kernel_of(act[j], blocks, split32 && act[j]->mm_f32) != key) continue;
                     used[j] = 1;
                     const Level *lv = level_of(act[j]);
                     if (lv) L.add(j, act[j]->d_mmt + lv->off, lv->n);
                 }
                 BLaunch b = finish(tb, L);
-                if (b.grid > 0) phases.push_back({b, act[i]->kid, f32});
+                if (b.grid > 0) phases.push_back({b, key.first, key.second});
             }
         };
         for (size_t k = 0; k < max_fwd; k++)
-            add_phase([&](h2p_hip_handle *h) { return k < h->mm_fwd_levels.size() ? &h->mm_fwd_levels[k] : (const Level *)nullptr; }, false);
-        add_phase([&](h2p_hip_handle *h) { return (const Level *)&h->mm_intmd; }, true);
+            add_phase([&](h2p_hip_handle *h) { return k < h->mm_fwd_levels.size() ? &h->mm_fwd_levels[k] : (const Level *)nullptr; }, false, false);
+        add_phase([&](h2p_hip_handle *h) { return (const Level *)&h->mm_intmd; }, true, true);
         for (size_t k = 0; k < max_bwd; k++)
-            add_phase([&](h2p_hip_handle *h) { return k < h->mm_bwd_levels.size() ? &h->mm_bwd_levels[k] : (const Level *)nullptr; }, false);
-        add_phase([&](h2p_hip_handle *h) { return (const Level *)&h->mm_leaf; }, false);
-        add_phase([&](h2p_hip_handle *h) { return h->mm_f32 ? (const Level *)&h->mm_leaf32 : (const Level *)nullptr; }, true);
+            add_phase([&](h2p_hip_handle *h) { return k < h->mm_bwd_levels.size() ? &h->mm_bwd_levels[k] : (const Level *)nullptr; }, false, false);
+        add_phase([&](h2p_hip_handle *h) { return (const Level *)&h->mm_leaf; }, true, false);
+        add_phase([&](h2p_hip_handle *h) { return h->mm_f32 ? (const Level *)&h->mm_leaf32 : (const Level *)nullptr; }, true, true);
         const char *dbase = nullptr;
         if ((rc = stage_tables(B, tb, s, &dbase))) return rc;
         const MMCtx *dctx = (const MMCtx *)(dbase + ctx_off);
@@ -2564,39 +2622,12 @@ int h2p_hip_matmul_batch(h2p_hip_batch *B, int n, h2p_hip_handle *const *hs, int
             hipLaunchKernelGGL(k_mm_gather_b, dim3(lg.grid), dim3(256), 0, s, (const BatchItem *)(dbase + lg.items_off),
                                lg.n_items, dctx);
         int max_nvp = 16;
-        for (const MMCtx &c : ctx) max_nvp = std::max(max_nvp, c.P.nvp);
-        const int ncls = nv_class(max_nvp);
+        for (const MMCtx &c : ctx) max_nvp = std::max(max_nvp, c.A.P.nvp);
         for (const MMLaunch &ph : phases) {
             const BatchItem *it = (const BatchItem *)(dbase + ph.b.items_off);
-            const dim3 grid(ph.b.grid), blk(256);
-            if (ph.f32) {
-                switch (ph.kid * 3 + ncls) {
-                    case KC * 3 + 0: hipLaunchKernelGGL((k_mm32_b<KC, MMVar<1, 16, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                    case KC * 3 + 1: hipLaunchKernelGGL((k_mm32_b<KC, MMVar<1, 32, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                    case KC * 3 + 2: hipLaunchKernelGGL((k_mm32_b<KC, MMVar<1, 64, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                    case KG * 3 + 0: hipLaunchKernelGGL((k_mm32_b<KG, MMVar<1, 16, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                    case KG * 3 + 1: hipLaunchKernelGGL((k_mm32_b<KG, MMVar<1, 32, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                    case KG * 3 + 2: hipLaunchKernelGGL((k_mm32_b<KG, MMVar<1, 64, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                    case KM * 3 + 0: hipLaunchKernelGGL((k_mm32_b<KM, MMVar<1, 16, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                    case KM * 3 + 1: hipLaunchKernelGGL((k_mm32_b<KM, MMVar<1, 32, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                    default: hipLaunchKernelGGL((k_mm32_b<KM, MMVar<1, 64, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                }
-                continue;
-            }
-            switch (ph.kid * 3 + ncls) {
-                case KC * 3 + 0: hipLaunchKernelGGL((k_mm_b<KC, 1, MMVar<1, 16, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                case KC * 3 + 1: hipLaunchKernelGGL((k_mm_b<KC, 1, MMVar<1, 32, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                case KC * 3 + 2: hipLaunchKernelGGL((k_mm_b<KC, 1, MMVar<1, 64, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                case KG * 3 + 0: hipLaunchKernelGGL((k_mm_b<KG, 1, MMVar<1, 16, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                case KG * 3 + 1: hipLaunchKernelGGL((k_mm_b<KG, 1, MMVar<1, 32, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                case KG * 3 + 2: hipLaunchKernelGGL((k_mm_b<KG, 1, MMVar<1, 64, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                case KM * 3 + 0: hipLaunchKernelGGL((k_mm_b<KM, 1, MMVar<1, 16, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                case KM * 3 + 1: hipLaunchKernelGGL((k_mm_b<KM, 1, MMVar<1, 32, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                case KM * 3 + 2: hipLaunchKernelGGL((k_mm_b<KM, 1, MMVar<1, 64, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                case KR * 3 + 0: hipLaunchKernelGGL((k_mm_b<KR, 3, MMVar<3, 16, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                case KR * 3 + 1: hipLaunchKernelGGL((k_mm_b<KR, 3, MMVar<3, 32, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-                default: hipLaunchKernelGGL((k_mm_b<KR, 3, MMVar<3, 64, 0>>), grid, blk, 0, s, it, ph.b.n_items, dctx); break;
-            }
+            if (max_nvp <= 16) launch_mm_b<1>(ph.kind, ph.kid, it, ph.b, dctx, s);
+            else if (max_nvp <= 32) launch_mm_b<2>(ph.kind, ph.kid, it, ph.b, dctx, s);
+            else launch_mm_b<4>(ph.kind, ph.kid, it, ph.b, dctx, s);
         }
         if (ls.grid > 0)
             hipLaunchKernelGGL(k_mm_scatter_b, dim3(ls.grid), dim3(256), 0, s, (const BatchItem *)(dbase + ls.items_off),

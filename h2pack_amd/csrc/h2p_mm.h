@@ -11,12 +11,32 @@
 //   downward : Y1[children] += U[node] * Y1[node]           (level by level)
 //   leaves   : PY[leaf rows] = U[leaf] * Y1[leaf] + sum op(D) * PX + sum op(B) * Y0
 // A_s is a dense block (U, U^T, or a stored B/D block, transposed for the
-// negative entries of the pair-to-block CSR) or, in JIT mode, kernel values
-// evaluated into the tile: the kernels are symmetric, so op(B) = K(dst set,
-// src set).  Panels are row-major with a row length of nvp (vectors padded to
-// a multiple of 16).  The products run on v_mfma_f64_16x16x4f64: lane l
-// supplies A[l % 16][l / 16] and B[l / 16][l % 16] and receives
-// D[4 r + l / 16][l % 16] in its register r.
+// negative entries of the pair-to-block CSR) or, in JIT mode, kernel values:
+// the kernels are symmetric, so op(B) = K(dst set, src set).  Panels are
+// row-major with a row length of nvp (vectors padded to a multiple of 16).
+//
+// Work split.  A destination is cut into tasks of MM_PIECE (32) rows, or 16
+// points = 48 rows for the evaluated 3x3 kernel; the four waves of a
+// workgroup share a task's rows and deal its inner entries round-robin in
+// chunks of 16 (4 points for the 3x3 kernel), and their four accumulator
+// sets are added in wave order at the end.  So a wave needs nothing from the
+// others before that: no barrier and no LDS staging in the inner loop, and
+// a task's longest chain is a quarter of its sources.
+//
+// Operands stay in registers.  v_mfma_f64_16x16x4f64: lane l supplies
+// A[l % 16][l / 16] and B[l / 16][l % 16] and receives D[4 r + l / 16][l % 16]
+// in register r.  Four such products consume 16 inner entries, and any
+// assignment of the 16 entries to (step, lane group) does, as long as A and X
+// use the same one:
+//   dense A    : step r, lane group g take entry 4 g + r, so a lane reads 32
+//                consecutive bytes of its row (transposed blocks: each step
+//                reads 16 consecutive rows' entries, 128 bytes per group);
+//   evaluated A: step r, lane group g take entry 4 r + g.  The tile of
+//                squared distances q[src][dst] of 16 sources x 16
+//                destinations is itself one MFMA whose result register r holds
+//                source 4 r + g against destination l % 16, exactly the A
+//                operand of step r: kernel values go from the evaluation into
+//                the product without leaving the lane.
 #pragma once
 #include "h2p_device.h"
 
@@ -25,21 +45,31 @@ namespace h2p {
 enum { MM_PX = 0, MM_Y0 = 1, MM_Y1 = 2, MM_PY = 3 };
 enum { MM_A_U = 0, MM_A_UT = 1, MM_A_BD = 2, MM_A_JIT = 3 };
 
+#define H2P_MM_MAXNVP 64
+#define H2P_MM_NVARIANT 4
+#define H2P_MM_PIECE 32       // rows of a task
+#define H2P_MM_PIECE3 48      // rows of a task with evaluated 3x3 blocks
+
+// One source block of a destination (shared by the destination's tasks).
 struct MMSrc {
-    long long a_off;   // dense: element offset of A in its blob
+    long long a_off;   // dense: element offset of op(A)'s first row in its blob
     int kind;          // MM_A_*
     int trans;         // dense: op(A) = A^T
     int lda;           // dense: row length of the stored A
     int K;             // inner dimension (vector entries)
-    int c0, c1;        // JIT: first destination / source point (unified coordinates)
+    int c1;            // JIT: first source point (unified coordinates)
     int x_space, x_off;
     int shift;         // JIT: shift-table entry added to the source points (periodic images)
-    int pad;
 };
 
+// M destination rows from row m0 of a destination; its sources in
+// [sbeg, smid) are dense, those in [smid, send) evaluated.
 struct MMTask {
     int dst_space, dst_off, M, accumulate;
-    int sbeg, send, pad0, pad1;
+    int sbeg, smid, send;
+    int m0;            // first row within the destination (dense sources' row offset)
+    int c0;            // JIT: first destination point of this task (unified coordinates)
+    int pad;
 };
 
 struct MMPanels {
@@ -47,232 +77,378 @@ struct MMPanels {
     int nvp;           // padded row length
 };
 
-// Tile geometry of one variant: RC rows of the destination per chunk (a
-// multiple of 16, and of 48 for the 3x3 kernel so tiles hold whole points),
-// KC inner entries per LDS stage, NV the widest panel the variant takes.
-// The (RC/16) x (nvp/16) output tiles of a chunk are dealt to the four waves
-// round-robin, so every wave issues MFMAs whatever the panel width.
-template <int RC_, int KC_, int NV_>
-struct MMCfg {
-    static constexpr int RC = RC_, KC = KC_, NV = NV_;
-    static_assert(RC % 16 == 0 && KC % 4 == 0 && NV % 16 == 0 && NV <= 64, "bad tile geometry");
+// the operands of a launch beside its tasks
+struct MMArgs {
+    const MMSrc *srcs;
+    const double *U, *UT;
+    const void *BD;            // stored blocks (double, or float for the FP32 products)
+    const double *cx;          // unified coordinates, one row per dimension
+    long long cstride;
+    const double *shifts;
+    double scale;              // coordinate scale of the FP64 norm-form kernels
+    KParam kp;
+    MMPanels P;
 };
 
-#define H2P_MM_MAXNVP 64
-#define H2P_MM_NVARIANT 4
+// x x + y y + z z with its roundings fixed, so that every kernel that forms a
+// kernel value gets the same bits
+__device__ __forceinline__ double mm_sq3(double x, double y, double z) {
+    return __builtin_fma(z, z, __builtin_fma(x, x, y * y));
+}
 
-// The variants the autotuner chooses from, per kernel dimension and panel
-// width class (NV = 16, 32, 64); variant 0 is the default.
-template <int KD, int NV, int V> struct MMVar;
-template <int NV> struct MMVar<1, NV, 0> : MMCfg<64, 32, NV> {};
-template <int NV> struct MMVar<1, NV, 1> : MMCfg<64, 64, NV> {};
-template <int NV> struct MMVar<1, NV, 2> : MMCfg<128, 32, NV> {};
-template <int NV> struct MMVar<1, NV, 3> : MMCfg<32, 64, NV> {};
-template <int NV> struct MMVar<3, NV, 0> : MMCfg<48, 48, NV> {};
-template <int NV> struct MMVar<3, NV, 1> : MMCfg<96, 24, NV> {};
-template <int NV> struct MMVar<3, NV, 2> : MMCfg<96, 48, NV> {};
-template <int NV> struct MMVar<3, NV, 3> : MMCfg<48, 24, NV> {};
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
-// One stage of a task: the (RC x KC) operator tile of source si at inner
-// offset kc and the (KC x nvp) operand tile, fetched into registers (loads
-// or kernel evaluations), then stored to LDS.  The stages of a chunk run as
-// a software pipeline: stage s + 1 is fetched before the MFMAs of stage s
-// are issued, so its global-memory latency (or its kernel evaluations)
-// overlaps the matrix work.
-template <int KID, int KD, class G>
-struct MMStage {
-    static constexpr int RC = G::RC, KC = G::KC, NV = G::NV;
-    // per thread: NA kernel-evaluated pairs (JIT; 9 entries each for the 3x3
-    // kernel) or ND stored entries (dense), NX operand entries
-    static constexpr int NA = ((RC / KD) * (KC / KD) + 255) / 256;
-    static constexpr int ND = (RC * KC + 255) / 256;
-    static constexpr int NX = (KC * NV + 255) / 256;
-    static constexpr int NREG = (KD * KD * NA > ND) ? KD * KD * NA : ND;
-    double a[NREG];
-    double x[NX];
-
-    __device__ __forceinline__ void fetch(const MMTask &t, const MMSrc &s, int mc, int kc, int nvp,
-                                          const double *__restrict__ Ublob, const double *__restrict__ UTblob,
-                                          const double *__restrict__ BDblob, const double *__restrict__ cx,
-                                          long long cstride, const KParam &kp,
-                                          const double *__restrict__ shifts, const MMPanels &P) {
-        // rows of cx: x, y, z and, for the 3x3 kernel, radius and reciprocal radius
-        const double *cy = cx + cstride, *cz = cx + 2 * cstride, *ca = cx + 3 * cstride, *cia = cx + 4 * cstride;
-        if (s.kind == MM_A_JIT) {
-            constexpr int RP = RC / KD, CP = KC / KD;
-            const int p0 = mc / KD, q0 = kc / KD;
-            const int np0 = t.M / KD - p0, nq0 = s.K / KD - q0;
-            const double hx = shifts[3 * s.shift], hy = shifts[3 * s.shift + 1], hz = shifts[3 * s.shift + 2];
-#pragma unroll
-            for (int u = 0; u < NA; u++) {
-                const int e = threadIdx.x + 256 * u;
-                const int i = e / CP, j = e - i * CP;
-                const bool ok = e < RP * CP && i < np0 && j < nq0;
-                const int gi = s.c0 + p0 + (ok ? i : 0), gj = s.c1 + q0 + (ok ? j : 0);
-                const double dx = cx[gi] - (cx[gj] + hx), dy = cy[gi] - (cy[gj] + hy), dz = cz[gi] - (cz[gj] + hz);
-                if constexpr (KD == 1) {
-                    a[u] = ok ? kval<KID>(dx * dx + dy * dy + dz * dz, kp) : 0.0;
-                } else {
-                    double t1, t2, ux, uy, uz;
-                    rpy_coef_rcp(dx, dy, dz, ca[gi], ca[gj], cia[gi], cia[gj], kp.p1, t1, t2, ux, uy, uz);
-                    const double uu[3] = {ux, uy, uz};
-#pragma unroll
-                    for (int p = 0; p < 3; p++)
-#pragma unroll
-                        for (int q = 0; q < 3; q++)
-                            a[9 * u + 3 * p + q] = ok ? t2 * uu[p] * uu[q] + (p == q ? t1 : 0.0) : 0.0;
-                }
-            }
-        } else {
-            const double *A = (s.kind == MM_A_U ? Ublob : s.kind == MM_A_UT ? UTblob : BDblob) + s.a_off;
-#pragma unroll
-            for (int u = 0; u < ND; u++) {
-                const int e = threadIdx.x + 256 * u;
-                int i, j;
-                if (!s.trans) { i = e / KC; j = e - i * KC; }      // consecutive lanes along a row of A
-                else { j = e / RC; i = e - j * RC; }              // consecutive lanes along a row of A^T
-                const int m = mc + i, k = kc + j;
-                const bool ok = e < RC * KC && m < t.M && k < s.K;
-                a[u] = ok ? (s.trans ? A[(long long)k * s.lda + m] : A[(long long)m * s.lda + k]) : 0.0;
-            }
-        }
-        const double *X = P.p[s.x_space] + (long long)s.x_off * nvp;
-#pragma unroll
-        for (int u = 0; u < NX; u++) {
-            const int e = threadIdx.x + 256 * u;
-            const int k = e / nvp, c = e - k * nvp;
-            x[u] = (e < KC * nvp && kc + k < s.K) ? X[(long long)(kc + k) * nvp + c] : 0.0;
+// Walks the chunks of a source list that belong to one wave: chunk indices
+// run through the sources one after the other and wave w takes w, w + 4, ...
+// All members are the same on every lane.
+template <int CH>
+struct MMCursor {
+    int si, c, nch, send;
+    MMSrc s;
+    __device__ __forceinline__ void settle(const MMSrc *__restrict__ srcs) {
+        while (c >= nch) {
+            c -= nch;
+            if (++si >= send) return;
+            s = srcs[si];
+            nch = (s.K + CH - 1) / CH;
         }
     }
-
-    __device__ __forceinline__ void store(const MMSrc &s, int nvp, double (*As)[KC + 1], double (*Xs)[NV + 1]) const {
-        if (s.kind == MM_A_JIT) {
-            constexpr int RP = RC / KD, CP = KC / KD;
-#pragma unroll
-            for (int u = 0; u < NA; u++) {
-                const int e = threadIdx.x + 256 * u;
-                if (e >= RP * CP) break;
-                const int i = e / CP, j = e - i * CP;
-                if constexpr (KD == 1) {
-                    As[i][j] = a[u];
-                } else {
-#pragma unroll
-                    for (int p = 0; p < 3; p++)
-#pragma unroll
-                        for (int q = 0; q < 3; q++) As[3 * i + p][3 * j + q] = a[9 * u + 3 * p + q];
-                }
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < ND; u++) {
-                const int e = threadIdx.x + 256 * u;
-                if (e >= RC * KC) break;
-                int i, j;
-                if (!s.trans) { i = e / KC; j = e - i * KC; }
-                else { j = e / RC; i = e - j * RC; }
-                As[i][j] = a[u];
-            }
+    __device__ __forceinline__ void start(const MMSrc *__restrict__ srcs, int beg, int end, int w) {
+        si = beg;
+        send = end;
+        c = w;
+        nch = 0;
+        if (si < send) {
+            s = srcs[si];
+            nch = (s.K + CH - 1) / CH;
+            settle(srcs);
         }
-#pragma unroll
-        for (int u = 0; u < NX; u++) {
-            const int e = threadIdx.x + 256 * u;
-            if (e >= KC * nvp) break;
-            const int k = e / nvp, c = e - k * nvp;
-            Xs[k][c] = x[u];
-        }
+    }
+    __device__ __forceinline__ bool live() const { return si < send; }
+    __device__ __forceinline__ void next(const MMSrc *__restrict__ srcs) {
+        c += 4;
+        settle(srcs);
     }
 };
 
-// the stage after (si, kc): next inner chunk, or the first chunk of the next
-// source with K > 0
-__device__ __forceinline__ void mm_next(const MMSrc *__restrict__ srcs, int send, int KCs, int &si, int &kc) {
-    kc += KCs;
-    if (kc < srcs[si].K) return;
-    kc = 0;
-    for (si++; si < send && srcs[si].K <= 0; si++) {}
+// Destination row of entry `lane row` i of tile t: consecutive rows, or for
+// the 3x3 kernel one tensor component of 16 points per tile.
+template <bool ROW3>
+__device__ __forceinline__ int mm_row(int t, int i) {
+    return ROW3 ? 3 * i + t : 16 * t + i;
 }
 
-template <int KID, int KD, class G>
-__device__ __forceinline__ void mm_body(const MMTask &t, const MMSrc *__restrict__ srcs,
-                                        const double *__restrict__ Ublob,
-                                        const double *__restrict__ UTblob,
-                                        const double *__restrict__ BDblob,
-                                        const double *__restrict__ cx, long long cstride,
-                                        const KParam &kp, const double *__restrict__ shifts,
-                                        const MMPanels &P) {
-    constexpr int RC = G::RC, KC = G::KC, NV = G::NV;
-    constexpr int MT = RC / 16;                         // M tiles per chunk
-    constexpr int SLOTS = (MT * (NV / 16) + 3) / 4;     // output tiles per wave, at most
-    __shared__ double As[RC][KC + 1];
-    __shared__ double Xs[KC][NV + 1];
-    const int nvp = P.nvp, NT = nvp >> 4;               // nvp <= NV (host-checked)
-    const int T = MT * NT;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int li = lane & 15, lq = lane >> 4;
-    double *dst = P.p[t.dst_space] + (long long)t.dst_off * nvp;
-    int s_first = t.sbeg;
-    while (s_first < t.send && srcs[s_first].K <= 0) s_first++;
-    MMStage<KID, KD, G> stg;
-    for (int mc = 0; mc < t.M; mc += RC) {
-        d4 acc[SLOTS];
+// A operand of one 16-entry chunk of a dense source: a[t][r] = op(A)[row][kc + 4 lg + r],
+// rows past the task's last repeat it, entries past K repeat the last.
+template <int MT, bool ROW3>
+__device__ __forceinline__ void mm_load_a(const double *__restrict__ blob, const MMSrc &s, int m0, int M, int kc,
+                                          int li, int lg, double (*a)[4]) {
+    const bool full = kc + 16 <= s.K;
 #pragma unroll
-        for (int j = 0; j < SLOTS; j++) acc[j] = (d4){0.0, 0.0, 0.0, 0.0};
-        int si = s_first, kc = 0;
-        if (si < t.send)
-            stg.fetch(t, srcs[si], mc, kc, nvp, Ublob, UTblob, BDblob, cx, cstride, kp, shifts, P);
-        while (si < t.send) {
-            const MMSrc cur = srcs[si];
-            __syncthreads();                 // the previous stage's MFMAs are done with LDS
-            stg.store(cur, nvp, As, Xs);
-            __syncthreads();
-            int nsi = si, nkc = kc;
-            mm_next(srcs, t.send, KC, nsi, nkc);
-            if (nsi < t.send)                // next stage in flight during the MFMAs
-                stg.fetch(t, srcs[nsi], mc, nkc, nvp, Ublob, UTblob, BDblob, cx, cstride, kp, shifts, P);
+    for (int t = 0; t < MT; t++) {
+        const int row = m0 + min(mm_row<ROW3>(t, li), M - 1);
+        if (!s.trans) {
+            const double *p = blob + s.a_off + (long long)row * s.lda + kc + 4 * lg;
+            if (full) {
+                const d2u u = *(const d2u *)p, v = *(const d2u *)(p + 2);
+                a[t][0] = u.x;
+                a[t][1] = u.y;
+                a[t][2] = v.x;
+                a[t][3] = v.y;
+            } else {
 #pragma unroll
-            for (int j = 0; j < SLOTS; j++) {
-                const int tt = w + 4 * j;
-                if (tt < T) {
-                    const int mt = tt / NT, nt = tt - mt * NT;
-#pragma unroll
-                    for (int kk = 0; kk < KC; kk += 4)
-                        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(As[mt * 16 + li][kk + lq],
-                                                                      Xs[kk + lq][nt * 16 + li], acc[j], 0, 0, 0);
-                }
+                for (int r = 0; r < 4; r++) a[t][r] = p[min(4 * lg + r, s.K - 1 - kc) - 4 * lg];
             }
-            si = nsi;
-            kc = nkc;
-        }
-        // ---- write the chunk: register r of lane (li, lq) holds row 4 r + lq
-        // of its M tile, column li (the f64 16x16x4 output layout)
+        } else {
+            const double *p = blob + s.a_off + row;
 #pragma unroll
-        for (int j = 0; j < SLOTS; j++) {
-            const int tt = w + 4 * j;
-            if (tt < T) {
-                const int mt = tt / NT, nt = tt - mt * NT;
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int m = mc + mt * 16 + 4 * r + lq;
-                    if (m < t.M) {
-                        double *o = dst + (long long)m * nvp + nt * 16 + li;
-                        *o = t.accumulate ? *o + acc[j][r] : acc[j][r];
-                    }
-                }
-            }
+            for (int r = 0; r < 4; r++) a[t][r] = p[(long long)min(kc + 4 * lg + r, s.K - 1) * s.lda];
         }
-        __syncthreads();                     // LDS reuse by the next chunk
     }
 }
 
-template <int KID, int KD, class G>
-__global__ void __launch_bounds__(256) k_mm(const MMTask *__restrict__ tasks,
-                                            const MMSrc *__restrict__ srcs,
-                                            const double *__restrict__ Ublob,
-                                            const double *__restrict__ UTblob,
-                                            const double *__restrict__ BDblob,
-                                            const double *__restrict__ cx, long long cstride,
-                                            KParam kp, const double *__restrict__ shifts, MMPanels P) {
-    mm_body<KID, KD, G>(tasks[blockIdx.x], srcs, Ublob, UTblob, BDblob, cx, cstride, kp, shifts, P);
+// X operand rows: x[r][n] = X[row(r)][16 n + li] with row(r) = kc + k0 + kr r,
+// zero past K.  NT column tiles of the panel are live (GUARD: fewer than
+// NVT may be).
+template <int NVT, bool GUARD>
+__device__ __forceinline__ void mm_load_x(const double *__restrict__ X, int nvp, int nt, int K, int kc, int k0, int kr,
+                                          int li, double (*x)[NVT]) {
+    const bool full = kc + 16 <= K;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int k = kc + k0 + kr * r;
+        const double *p = X + (long long)(full ? k : min(k, K - 1)) * nvp + li;
+#pragma unroll
+        for (int n = 0; n < NVT; n++) {
+            if (GUARD && n >= nt) continue;
+            const double v = p[16 * n];
+            x[r][n] = (full || k < K) ? v : 0.0;
+        }
+    }
+}
+
+// The dense sources [sbeg, send) of a task: a software pipeline over the
+// wave's chunks, the next chunk's operands in flight during the products.
+template <int MT, bool ROW3, int NVT, bool GUARD>
+__device__ __forceinline__ void mm_dense(const MMTask &t, int sbeg, int send, const MMArgs &A, int nt, int w, int li,
+                                         int lg, d4 (*acc)[NVT]) {
+    MMCursor<16> cu;
+    cu.start(A.srcs, sbeg, send, w);
+    if (!cu.live()) return;
+    double a[MT][4], x[4][NVT];
+    auto fetch = [&](const MMSrc &s, int c) {
+        const double *blob = s.kind == MM_A_U ? A.U : s.kind == MM_A_UT ? A.UT : (const double *)A.BD;
+        mm_load_a<MT, ROW3>(blob, s, t.m0, t.M, 16 * c, li, lg, a);
+        const double *X = A.P.p[s.x_space] + (long long)s.x_off * A.P.nvp;
+        mm_load_x<NVT, GUARD>(X, A.P.nvp, nt, s.K, 16 * c, 4 * lg, 1, li, x);
+    };
+    fetch(cu.s, cu.c);
+    while (cu.live()) {
+        double a0[MT][4], x0[4][NVT];
+#pragma unroll
+        for (int q = 0; q < MT; q++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) a0[q][r] = a[q][r];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int n = 0; n < NVT; n++) x0[r][n] = x[r][n];
+        cu.next(A.srcs);
+        if (cu.live()) fetch(cu.s, cu.c);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int n = 0; n < NVT; n++) {
+                if (GUARD && n >= nt) continue;
+#pragma unroll
+                for (int q = 0; q < MT; q++)
+                    acc[q][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[q][r], x0[r][n], acc[q][n], 0, 0, 0);
+            }
+    }
+}
+
+// The evaluated sources of a task, scalar kernels: 16 sources x 32
+// destinations per chunk, distances by MFMA (Gaussian, Matern; coordinates
+// relative to the task's first destination point, pre-scaled as in the
+// matvec) or from coordinate differences (Coulomb, whose r = 0 must be
+// exact), kernel values straight into the products.
+template <int KID, int NVT, bool GUARD>
+__device__ __forceinline__ void mm_jit1(const MMTask &t, const MMArgs &A, int nt, int w, int li, int lg,
+                                        const double *e2t, d4 (*acc)[NVT]) {
+    constexpr bool NORM = KID != KC;
+    const double *cx = A.cx, *cy = A.cx + A.cstride, *cz = A.cx + 2 * A.cstride;
+    const double scale = A.scale, diag = A.kp.p0;
+    const double ox = NORM ? cx[t.c0] : 0.0, oy = NORM ? cy[t.c0] : 0.0, oz = NORM ? cz[t.c0] : 0.0;
+    MMCursor<16> cu;
+    cu.start(A.srcs, t.smid, t.send, w);
+    if (!cu.live()) return;
+    // destinations of the two tiles: point 16 q + li (the B operand (1, r)
+    // and the accumulator input |r|^2, or the plain coordinates)
+    double db[2], dx[2], dy[2], dz[2];
+    d4 dn[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int g = t.c0 + min(16 * q + li, t.M - 1);
+        dx[q] = (cx[g] - ox) * scale;
+        dy[q] = (cy[g] - oy) * scale;
+        dz[q] = (cz[g] - oz) * scale;
+        const double nn = mm_sq3(dx[q], dy[q], dz[q]);
+        dn[q] = (d4){nn, nn, nn, nn};
+        db[q] = lg == 0 ? 1.0 : lg == 1 ? dx[q] : lg == 2 ? dy[q] : dz[q];
+    }
+    // sources of a chunk: point li (norm form) or points 4 r + lg
+    constexpr int NC = NORM ? 1 : 4;
+    double sx[NC], sy[NC], sz[NC];
+    auto fetch = [&](const MMSrc &s, int c) {
+#pragma unroll
+        for (int r = 0; r < NC; r++) {
+            const int g = s.c1 + min(16 * c + (NORM ? li : 4 * r + lg), s.K - 1);
+            sx[r] = cx[g];
+            sy[r] = cy[g];
+            sz[r] = cz[g];
+        }
+    };
+    fetch(cu.s, cu.c);
+    const bool two = t.M > 16;
+    while (cu.live()) {
+        double x[4][NVT];
+        mm_load_x<NVT, GUARD>(A.P.p[cu.s.x_space] + (long long)cu.s.x_off * A.P.nvp, A.P.nvp, nt, cu.s.K, 16 * cu.c,
+                              lg, 4, li, x);
+        double px[NC], py[NC], pz[NC];
+#pragma unroll
+        for (int r = 0; r < NC; r++) {
+            px[r] = sx[r];
+            py[r] = sy[r];
+            pz[r] = sz[r];
+        }
+        cu.next(A.srcs);
+        if (cu.live()) fetch(cu.s, cu.c);
+        double sa = 0.0;
+        if constexpr (NORM) {
+            const double ux = (px[0] - ox) * scale, uy = (py[0] - oy) * scale, uz = (pz[0] - oz) * scale;
+            const double nn = mm_sq3(ux, uy, uz);
+            sa = lg == 0 ? nn : -2.0 * (lg == 1 ? ux : lg == 2 ? uy : uz);
+        }
+        auto tile = [&](int q) {
+            d4 d2;
+            if constexpr (NORM) d2 = __builtin_amdgcn_mfma_f64_16x16x4f64(sa, db[q], dn[q], 0, 0, 0);
+            double kv[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if constexpr (NORM) {
+                    kv[r] = kprep<KID>(d2[r], diag, e2t);
+                } else {
+                    const double ex = dx[q] - px[r], ey = dy[q] - py[r], ez = dz[q] - pz[r];
+                    kv[r] = kprep<KID>(mm_sq3(ex, ey, ez), diag);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int n = 0; n < NVT; n++) {
+                    if (GUARD && n >= nt) continue;
+                    acc[q][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(kv[r], x[r][n], acc[q][n], 0, 0, 0);
+                }
+        };
+        tile(0);
+        if (two) tile(1);
+    }
+}
+
+// The evaluated sources of a task, 3x3 kernel: 4 source points x 16
+// destination points per chunk.  Lane l evaluates the pair (destination
+// l % 16, source l / 16) once; its six distinct tensor entries are the A
+// operands of nine products, one per component pair.
+template <int NVT, bool GUARD>
+__device__ __forceinline__ void mm_jit3(const MMTask &t, const MMArgs &A, int nt, int w, int li, int lg,
+                                        d4 (*acc)[NVT]) {
+    const double *cx = A.cx;
+    const long long cs = A.cstride;
+    MMCursor<12> cu;
+    cu.start(A.srcs, t.smid, t.send, w);
+    if (!cu.live()) return;
+    double d[5], sp[5];
+    {
+        const int g = t.c0 + min(li, t.M / 3 - 1);
+#pragma unroll
+        for (int k = 0; k < 5; k++) d[k] = cx[k * cs + g];
+    }
+    auto fetch = [&](const MMSrc &s, int c) {
+        const int g = s.c1 + min(4 * c + lg, s.K / 3 - 1);
+#pragma unroll
+        for (int k = 0; k < 5; k++) sp[k] = cx[k * cs + g];
+#pragma unroll
+        for (int k = 0; k < 3; k++) sp[k] += A.shifts[3 * s.shift + k];
+    };
+    fetch(cu.s, cu.c);
+    while (cu.live()) {
+        double x[3][NVT];
+        {
+            const int np = cu.s.K / 3, p = 4 * cu.c + lg;
+            const double *X = A.P.p[cu.s.x_space] + (long long)(cu.s.x_off + 3 * min(p, np - 1)) * A.P.nvp + li;
+#pragma unroll
+            for (int b = 0; b < 3; b++)
+#pragma unroll
+                for (int n = 0; n < NVT; n++) {
+                    if (GUARD && n >= nt) continue;
+                    const double v = X[(long long)b * A.P.nvp + 16 * n];
+                    x[b][n] = p < np ? v : 0.0;
+                }
+        }
+        const double ex = d[0] - sp[0], ey = d[1] - sp[1], ez = d[2] - sp[2], ra = sp[3], rb = sp[4];
+        cu.next(A.srcs);
+        if (cu.live()) fetch(cu.s, cu.c);
+        double t1, t2, ux, uy, uz;
+        rpy_coef_rcp(ex, ey, ez, d[3], ra, d[4], rb, A.kp.p1, t1, t2, ux, uy, uz);
+        const double gx = t2 * ux, gy = t2 * uy, gz = t2 * uz;
+        const double kxx = gx * ux + t1, kxy = gx * uy, kxz = gx * uz, kyy = gy * uy + t1, kyz = gy * uz,
+                     kzz = gz * uz + t1;
+        const double k3[3][3] = {{kxx, kxy, kxz}, {kxy, kyy, kyz}, {kxz, kyz, kzz}};
+#pragma unroll
+        for (int b = 0; b < 3; b++)
+#pragma unroll
+            for (int n = 0; n < NVT; n++) {
+                if (GUARD && n >= nt) continue;
+#pragma unroll
+                for (int a = 0; a < 3; a++)
+                    acc[a][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(k3[a][b], x[b][n], acc[a][n], 0, 0, 0);
+            }
+    }
+}
+
+// Adds the four waves' accumulators in wave order, a column tile at a time
+// through LDS (3 MT x 256 doubles), and writes the task's rows.
+template <int MT, bool ROW3, int NVT, bool GUARD>
+__device__ __forceinline__ void mm_finish(const MMTask &t, const MMPanels &P, int nt, int w, int lane, d4 (*acc)[NVT],
+                                          d4 *lds) {
+    double *dst = P.p[t.dst_space] + (long long)t.dst_off * P.nvp;
+    const int li = lane & 15, lg = lane >> 4;
+#pragma unroll
+    for (int n = 0; n < NVT; n++) {
+        if (GUARD && n >= nt) continue;
+        if (n > 0) __syncthreads();
+        if (w > 0)
+#pragma unroll
+            for (int q = 0; q < MT; q++) lds[((w - 1) * MT + q) * H2P_WAVE + lane] = acc[q][n];
+        __syncthreads();
+        if (w > 0) continue;
+#pragma unroll
+        for (int q = 0; q < MT; q++) {
+            d4 v = acc[q][n];
+#pragma unroll
+            for (int k = 0; k < 3; k++) v += lds[(k * MT + q) * H2P_WAVE + lane];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int m = mm_row<ROW3>(q, 4 * r + lg);
+                if (m < t.M) {
+                    double *o = dst + (long long)m * P.nvp + 16 * n + li;
+                    *o = t.accumulate ? *o + v[r] : v[r];
+                }
+            }
+        }
+    }
+}
+
+// Dense tasks (U phases, stored blocks).
+template <int NVT, bool GUARD>
+__device__ __forceinline__ void mmd_body(const MMTask &t, const MMArgs &A) {
+    __shared__ d4 lds[3 * 2 * H2P_WAVE];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nt = GUARD ? A.P.nvp >> 4 : NVT;
+    d4 acc[2][NVT];
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int n = 0; n < NVT; n++) acc[q][n] = (d4){0.0, 0.0, 0.0, 0.0};
+    mm_dense<2, false, NVT, GUARD>(t, t.sbeg, t.smid, A, nt, w, lane & 15, lane >> 4, acc);
+    mm_finish<2, false, NVT, GUARD>(t, A.P, nt, w, lane, acc, lds);
+}
+
+// Tasks with evaluated sources (after any dense ones).
+template <int KID, int NVT, bool GUARD>
+__device__ __forceinline__ void mmj_body(const MMTask &t, const MMArgs &A) {
+    constexpr bool R3 = KID == KR;
+    constexpr int MT = R3 ? 3 : 2;
+    __shared__ d4 lds[3 * MT * H2P_WAVE];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nt = GUARD ? A.P.nvp >> 4 : NVT;
+    d4 acc[MT][NVT];
+#pragma unroll
+    for (int q = 0; q < MT; q++)
+#pragma unroll
+        for (int n = 0; n < NVT; n++) acc[q][n] = (d4){0.0, 0.0, 0.0, 0.0};
+    if (t.smid > t.sbeg) mm_dense<MT, R3, NVT, GUARD>(t, t.sbeg, t.smid, A, nt, w, lane & 15, lane >> 4, acc);
+    if constexpr (R3) {
+        mm_jit3<NVT, GUARD>(t, A, nt, w, lane & 15, lane >> 4, acc);
+    } else if constexpr (KID == KC) {
+        mm_jit1<KID, NVT, GUARD>(t, A, nt, w, lane & 15, lane >> 4, nullptr, acc);
+    } else {
+        __shared__ double e2t[H2P_E2_N];
+        if (threadIdx.x < H2P_E2_N) e2t[threadIdx.x] = c_e2tab[threadIdx.x];
+        __syncthreads();
+        mm_jit1<KID, NVT, GUARD>(t, A, nt, w, lane & 15, lane >> 4, e2t, acc);
+    }
+    mm_finish<MT, R3, NVT, GUARD>(t, A.P, nt, w, lane, acc, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -283,164 +459,141 @@ __global__ void __launch_bounds__(256) k_mm(const MMTask *__restrict__ tasks,
 // operand rows rounded to FP32 run on v_mfma_f32_16x16x4f32; the FP32 tile
 // sums of every 16 inner entries (four products, counted from the start of
 // each source) are folded into FP64 accumulators, and the output panels
-// stay FP64.  The fold points do not depend on the tile variant (KC is a
-// multiple of 16), so every variant gives bitwise the same result.  The U phases keep the FP64 kernel.  Only
-// B/D sources reach this kernel (the host splits the leaf tasks into a U
-// part and a B/D part).
+// stay FP64.  The U phases keep the FP64 kernel.  Only B/D sources reach
+// this kernel (the host splits the leaf tasks into a U part and a B/D part).
 //
 // Lane layouts: v_mfma_f32_16x16x4f32 takes A[l % 16][l / 16] and
 // B[l / 16][l % 16] like the FP64 product, but returns D[4 (l / 16) + r]
 // [l % 16] in register r, where the FP64 product returns row 4 r + l / 16.
 // Feeding the A rows in the order sigma(4 a + b) = 4 b + a makes the FP32
 // tile land in the FP64 accumulator layout, so the fold is lane-local.
+// Inner entry of step r, lane group g: 4 r + g for both kinds of source.
 __device__ __forceinline__ int mm32_sigma(int i) { return 4 * (i & 3) + (i >> 2); }
 
-template <int KID, class G>
-struct MMStage32 {
-    static constexpr int RC = G::RC, KC = G::KC, NV = G::NV;
-    static_assert(KC % 16 == 0, "FP32 stages fold every 16 inner entries");
-    static constexpr int NA = (RC * KC + 255) / 256;
-    static constexpr int NX = (KC * NV + 255) / 256;
-    float a[NA];
-    float x[NX];
-
-    __device__ __forceinline__ void fetch(const MMTask &t, const MMSrc &s, int mc, int kc, int nvp,
-                                          const float *__restrict__ BD32, const double *__restrict__ cx,
-                                          long long cstride, float p0, const double *__restrict__ shifts,
-                                          const MMPanels &P) {
-        const double *cy = cx + cstride, *cz = cx + 2 * cstride;
-        if (s.kind == MM_A_JIT) {
-            const int np0 = t.M - mc, nq0 = s.K - kc;
-            const double hx = shifts[3 * s.shift], hy = shifts[3 * s.shift + 1], hz = shifts[3 * s.shift + 2];
+template <int KID, int NVT, bool GUARD>
+__device__ __forceinline__ void mm32_body(const MMTask &t, const MMArgs &A) {
+    __shared__ d4 lds[3 * 2 * H2P_WAVE];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lg = lane >> 4, ls = mm32_sigma(li);
+    const int nt = GUARD ? A.P.nvp >> 4 : NVT;
+    d4 acc[2][NVT];
 #pragma unroll
-            for (int u = 0; u < NA; u++) {
-                const int e = threadIdx.x + 256 * u;
-                const int i = e / KC, j = e - i * KC;
-                const bool ok = e < RC * KC && i < np0 && j < nq0;
-                const int gi = s.c0 + mc + (ok ? i : 0), gj = s.c1 + kc + (ok ? j : 0);
-                const double dx = cx[gi] - (cx[gj] + hx), dy = cy[gi] - (cy[gj] + hy), dz = cz[gi] - (cz[gj] + hz);
-                const double r2 = dx * dx + dy * dy + dz * dz;
-                a[u] = ok ? kvalf<KID>((float)r2, p0) : 0.0f;
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int n = 0; n < NVT; n++) acc[q][n] = (d4){0.0, 0.0, 0.0, 0.0};
+    const double *cx = A.cx, *cy = A.cx + A.cstride, *cz = A.cx + 2 * A.cstride;
+    const float p0 = (float)A.kp.p0;
+    const bool two = t.M > 16;
+    MMCursor<16> cu;
+    cu.start(A.srcs, t.sbeg, t.send, w);
+    // the next chunk's coordinates (JIT, KID >= 0) or block entries (KID < 0)
+    double dx[2], dy[2], dz[2], sx[4], sy[4], sz[4];
+    float a[2][4];
+    auto fetch = [&](const MMSrc &s, int c) {
+        if constexpr (KID >= 0) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int g = s.c1 + min(16 * c + 4 * r + lg, s.K - 1);
+                sx[r] = cx[g];
+                sy[r] = cy[g];
+                sz[r] = cz[g];
             }
         } else {
-            const float *A = BD32 + s.a_off;
 #pragma unroll
-            for (int u = 0; u < NA; u++) {
-                const int e = threadIdx.x + 256 * u;
-                int i, j;
-                if (!s.trans) { i = e / KC; j = e - i * KC; }
-                else { j = e / RC; i = e - j * RC; }
-                const int m = mc + i, k = kc + j;
-                const bool ok = e < RC * KC && m < t.M && k < s.K;
-                a[u] = ok ? (s.trans ? A[(long long)k * s.lda + m] : A[(long long)m * s.lda + k]) : 0.0f;
-            }
-        }
-        const double *X = P.p[s.x_space] + (long long)s.x_off * nvp;
-#pragma unroll
-        for (int u = 0; u < NX; u++) {
-            const int e = threadIdx.x + 256 * u;
-            const int k = e / nvp, c = e - k * nvp;
-            x[u] = (e < KC * nvp && kc + k < s.K) ? (float)X[(long long)(kc + k) * nvp + c] : 0.0f;
-        }
-    }
-
-    __device__ __forceinline__ void store(const MMSrc &s, int nvp, float (*As)[KC + 1], float (*Xs)[NV + 1]) const {
-#pragma unroll
-        for (int u = 0; u < NA; u++) {
-            const int e = threadIdx.x + 256 * u;
-            if (e >= RC * KC) break;
-            int i, j;
-            if (s.kind == MM_A_JIT || !s.trans) { i = e / KC; j = e - i * KC; }
-            else { j = e / RC; i = e - j * RC; }
-            As[i][j] = a[u];
-        }
-#pragma unroll
-        for (int u = 0; u < NX; u++) {
-            const int e = threadIdx.x + 256 * u;
-            if (e >= KC * nvp) break;
-            const int k = e / nvp, c = e - k * nvp;
-            Xs[k][c] = x[u];
-        }
-    }
-};
-
-template <int KID, class G>
-__device__ __forceinline__ void mm32_body(const MMTask &t, const MMSrc *__restrict__ srcs,
-                                          const float *__restrict__ BD32, const double *__restrict__ cx,
-                                          long long cstride, float p0, const double *__restrict__ shifts,
-                                          const MMPanels &P) {
-    constexpr int RC = G::RC, KC = G::KC, NV = G::NV;
-    constexpr int MT = RC / 16;
-    constexpr int SLOTS = (MT * (NV / 16) + 3) / 4;
-    __shared__ float As[RC][KC + 1];
-    __shared__ float Xs[KC][NV + 1];
-    const int nvp = P.nvp, NT = nvp >> 4;
-    const int T = MT * NT;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int li = lane & 15, lq = lane >> 4, ls = mm32_sigma(li);
-    double *dst = P.p[t.dst_space] + (long long)t.dst_off * nvp;
-    int s_first = t.sbeg;
-    while (s_first < t.send && srcs[s_first].K <= 0) s_first++;
-    MMStage32<KID, G> stg;
-    for (int mc = 0; mc < t.M; mc += RC) {
-        d4 acc[SLOTS];
-#pragma unroll
-        for (int j = 0; j < SLOTS; j++) acc[j] = (d4){0.0, 0.0, 0.0, 0.0};
-        int si = s_first, kc = 0;
-        if (si < t.send) stg.fetch(t, srcs[si], mc, kc, nvp, BD32, cx, cstride, p0, shifts, P);
-        while (si < t.send) {
-            const MMSrc cur = srcs[si];
-            __syncthreads();
-            stg.store(cur, nvp, As, Xs);
-            __syncthreads();
-            int nsi = si, nkc = kc;
-            mm_next(srcs, t.send, KC, nsi, nkc);
-            if (nsi < t.send) stg.fetch(t, srcs[nsi], mc, nkc, nvp, BD32, cx, cstride, p0, shifts, P);
-#pragma unroll
-            for (int j = 0; j < SLOTS; j++) {
-                const int tt = w + 4 * j;
-                if (tt < T) {
-                    const int mt = tt / NT, nt = tt - mt * NT;
-#pragma unroll
-                    for (int k0 = 0; k0 < KC; k0 += 16) {
-                        f4 a32 = (f4){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                        for (int kk = k0; kk < k0 + 16; kk += 4)
-                            a32 = __builtin_amdgcn_mfma_f32_16x16x4f32(As[mt * 16 + ls][kk + lq],
-                                                                       Xs[kk + lq][nt * 16 + li], a32, 0, 0, 0);
-#pragma unroll
-                        for (int r = 0; r < 4; r++) acc[j][r] += (double)a32[r];
-                    }
-                }
-            }
-            si = nsi;
-            kc = nkc;
-        }
-#pragma unroll
-        for (int j = 0; j < SLOTS; j++) {
-            const int tt = w + 4 * j;
-            if (tt < T) {
-                const int mt = tt / NT, nt = tt - mt * NT;
+            for (int q = 0; q < 2; q++) {
+                const int row = t.m0 + min(16 * q + ls, t.M - 1);
+                const float *p = (const float *)A.BD + s.a_off;
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const int m = mc + mt * 16 + 4 * r + lq;
-                    if (m < t.M) {
-                        double *o = dst + (long long)m * nvp + nt * 16 + li;
-                        *o = t.accumulate ? *o + acc[j][r] : acc[j][r];
-                    }
+                    const int k = min(16 * c + 4 * r + lg, s.K - 1);
+                    a[q][r] = s.trans ? p[(long long)k * s.lda + row] : p[(long long)row * s.lda + k];
                 }
             }
         }
-        __syncthreads();
+    };
+    if constexpr (KID >= 0) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const int g = t.c0 + min(16 * q + ls, t.M - 1);
+            dx[q] = cx[g];
+            dy[q] = cy[g];
+            dz[q] = cz[g];
+        }
     }
+    if (cu.live()) fetch(cu.s, cu.c);
+    while (cu.live()) {
+        double xd[4][NVT];
+        mm_load_x<NVT, GUARD>(A.P.p[cu.s.x_space] + (long long)cu.s.x_off * A.P.nvp, A.P.nvp, nt, cu.s.K, 16 * cu.c,
+                              lg, 4, li, xd);
+        double px[4], py[4], pz[4];
+        float a0[2][4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            if constexpr (KID >= 0) {
+                px[r] = sx[r];
+                py[r] = sy[r];
+                pz[r] = sz[r];
+            } else {
+                a0[0][r] = a[0][r];
+                a0[1][r] = a[1][r];
+            }
+        }
+        cu.next(A.srcs);
+        if (cu.live()) fetch(cu.s, cu.c);
+        float x[4][NVT];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int n = 0; n < NVT; n++) {
+                if (GUARD && n >= nt) continue;
+                x[r][n] = (float)xd[r][n];
+            }
+        auto tile = [&](int q) {
+            float kv[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if constexpr (KID >= 0) {
+                    const double ex = dx[q] - px[r], ey = dy[q] - py[r], ez = dz[q] - pz[r];
+                    const double r2 = mm_sq3(ex, ey, ez);
+                    kv[r] = kvalf<KID>((float)r2, p0);
+                } else {
+                    kv[r] = a0[q][r];
+                }
+            }
+#pragma unroll
+            for (int n = 0; n < NVT; n++) {
+                if (GUARD && n >= nt) continue;
+                f4 a32 = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int r = 0; r < 4; r++) a32 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[r], x[r][n], a32, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[q][n][r] += (double)a32[r];
+            }
+        };
+        tile(0);
+        if (two) tile(1);
+    }
+    mm_finish<2, false, NVT, GUARD>(t, A.P, nt, w, lane, acc, lds);
 }
 
-template <int KID, class G>
-__global__ void __launch_bounds__(256) k_mm32(const MMTask *__restrict__ tasks, const MMSrc *__restrict__ srcs,
-                                              const float *__restrict__ BD32, const double *__restrict__ cx,
-                                              long long cstride, float p0, const double *__restrict__ shifts,
-                                              MMPanels P) {
-    mm32_body<KID, G>(tasks[blockIdx.x], srcs, BD32, cx, cstride, p0, shifts, P);
+template <int NVT>
+__global__ void __launch_bounds__(256) k_mmd(const MMTask *__restrict__ tasks, MMArgs A) {
+    mmd_body<NVT, false>(tasks[blockIdx.x], A);
+}
+
+template <int KID, int NVT>
+__global__ void __launch_bounds__(256) k_mmj(const MMTask *__restrict__ tasks, MMArgs A) {
+    mmj_body<KID, NVT, false>(tasks[blockIdx.x], A);
+}
+
+// One column tile: 104 VGPRs by the compiler's own choice (4 waves per SIMD);
+// five waves hide the operand loads better (Matern N = 105k x8: 3.90 -> 3.80
+// ms).  Asking for a wave more of the wider or the FP64 builds spills and
+// measured slower (Coulomb N = 80k x20 2.52 -> 4.89 ms).
+template <int KID, int NVT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NVT == 1 ? 5 : 1, 8)))
+k_mm32(const MMTask *__restrict__ tasks, MMArgs A) {
+    mm32_body<KID, NVT, false>(tasks[blockIdx.x], A);
 }
 
 // Caller panel (original order, row- or column-major, ld) -> PX (permuted,

@@ -170,7 +170,7 @@ class H2MatHIP:
 
     def autotune(self, n_vec: int) -> dict:
         """Time the kernel variants on this matrix and keep the fastest
-        (h2p_hip_autotune): the matmul tiles per phase for ``n_vec`` columns,
+        (h2p_hip_autotune): the matmul task order per phase for ``n_vec`` columns,
         or with ``n_vec`` = 0 the matvec's grouped block launch, whether its
         D blocks run beside the sweeps (``d_concurrent``) and whether the
         levels above the leaf level run as a chain of their own beside the
@@ -188,7 +188,7 @@ class H2MatHIP:
         return out
 
     def mm_variant(self, phase: int, n_vec: int, variant: int = -1) -> int:
-        """Pin (variant >= 0) or read (variant -1) a matmul phase's tile variant."""
+        """Pin (variant >= 0) or read (variant -1) a matmul phase's variant."""
         rc = self.lib.h2p_hip_mm_variant(self.handle, int(phase), int(n_vec), int(variant))
         if rc < 0:
             _check(rc)

@@ -173,7 +173,7 @@ int h2p_hip_matmul_dev(h2p_hip_handle *h, int layout, int n_vec,
 /* h2p_hip_matmul_dev without any allocation.  No counterpart in the
  * reference: this is for callers that cannot allocate device memory during
  * the call (code under HIP graph capture, tight serving loops, harnesses
- * that forbid hipMalloc).  The same kernels and tile variants as
+ * that forbid hipMalloc).  The same kernels and variants as
  * h2p_hip_matmul_dev, bitwise the same result, launched directly (no
  * graph); the panels (permuted X, skeleton coefficients, permuted Y) live
  * in one static device array of H2P_HIP_NOALLOC_BYTES per GPU instead of
@@ -186,15 +186,16 @@ int h2p_hip_matmul_dev_noalloc(h2p_hip_handle *h, int layout, int n_vec,
                                const double *d_X, int ldx, double *d_Y,
                                int ldy, void *stream);
 
-/* Autotuner of the matmul tiles.  Each matmul phase (upward sweep, coupling,
- * downward sweep, leaf outputs) runs as grouped MFMA launches whose tile
- * geometry (rows per chunk, inner entries per LDS stage) is one of
- * H2P_HIP_MM_VARIANTS compiled variants.  This call times every variant on
- * the handle's own blocks for panels of n_vec columns and keeps the fastest
- * per phase; choices are shared, within the process, by handles whose phase
- * has the same kernel, mode and block-size histogram.  Every variant
- * computes bitwise the same result.  Optional outputs: summed phase times
- * of the default variants and of the chosen ones, in milliseconds.
+/* Autotuner of the matmul's task orders.  Each matmul phase (upward sweep,
+ * coupling, downward sweep, leaf outputs) runs as grouped MFMA launches of
+ * tasks in one of two orders: the tasks of a destination on one XCD (even
+ * variants, the default) or the longest tasks first (odd variants).  This
+ * call times both on the handle's own blocks for panels of n_vec columns and
+ * keeps the faster per phase; choices are shared, within the process, by
+ * handles whose phase has the same kernel, mode and block-size histogram.
+ * Every variant computes bitwise the same result.  Optional outputs: summed
+ * phase times of the default variants and of the chosen ones, in
+ * milliseconds.
  * n_vec = 0 tunes the matvec instead: its grouped B/D launch has two
  * builds of the same body compiled for different occupancies (JIT: 4 waves
  * per SIMD by default, unconstrained registers as the alternative; AOT:
@@ -207,7 +208,7 @@ int h2p_hip_matmul_dev_noalloc(h2p_hip_handle *h, int layout, int n_vec,
 int h2p_hip_autotune(h2p_hip_handle *h, int n_vec, double *t_default_ms,
                      double *t_tuned_ms);
 
-/* Pin the tile variant (0 .. H2P_HIP_MM_VARIANTS-1) of one matmul phase
+/* Pin the variant (0 .. H2P_HIP_MM_VARIANTS-1) of one matmul phase
  * (0..3, or -1 for all) for panels of n_vec columns; variant -1 returns the
  * current choice of the phase (phase -1: of phase 0) instead.  Phase 4 is
  * the matvec's block launch (variants 0 and 1; n_vec is ignored), phase 5
