@@ -84,13 +84,21 @@ k_blocks_jit2_b(const BatchItem *__restrict__ items, int n, const ReqCtx *__rest
                              c.coord, c.CT, c.scale, c.diag, c.xin, c.arena);
 }
 
-template <int KID, int KD, typename T = double>
-__global__ void __launch_bounds__(256) k_blocks_jit_b(const BatchItem *__restrict__ items, int n,
-                                                      const ReqCtx *__restrict__ reqs) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_blocks_rpy_b(const BatchItem *__restrict__ items, int n, const ReqCtx *__restrict__ reqs) {
+    const int it = find_item(items, n, blockIdx.x);
+    const ReqCtx &c = reqs[items[it].req];
+    const BatchItem &I = items[it];
+    blocks_rpy_unit<false>((const BlkTask *)I.tasks, blockIdx.x - I.begin, I.nbig, I.ntask, c.coord, c.CT, c.kp.p1,
+                           c.shifts, c.xin, c.arena);
+}
+
+__global__ void __launch_bounds__(256) k_blocks_rpy32_b(const BatchItem *__restrict__ items, int n,
+                                                        const ReqCtx *__restrict__ reqs) {
     const int it = find_item(items, n, blockIdx.x);
     const ReqCtx &c = reqs[items[it].req];
     const BlkTask t = ((const BlkTask *)items[it].tasks)[blockIdx.x - items[it].begin];
-    blocks_jit_body<KID, KD, T>(t, c.coord, c.CT, c.kp, c.shifts, c.xin, c.arena);
+    blocks_rpy32(t, c.coord, c.CT, c.kp, c.shifts, c.xin, c.arena);
 }
 
 template <typename TS>

@@ -222,14 +222,17 @@ static void free_handle(h2p_hip_handle *h) {
     delete h;
 }
 
-template <int KID, int KD>
-static void launch_jit(h2p_hip_handle *h, hipStream_t s) {
+static void launch_rpy(h2p_hip_handle *h, hipStream_t s) {
+    const auto &P = h->part[0];
     if (h->prec == H2P_HIP_FP32MIX)
-        hipLaunchKernelGGL((k_blocks_jit<KID, KD, float>), dim3(h->n_blk), dim3(256), 0, s, h->d_blk,
-                           h->d_coord, h->CT, h->kp, h->d_shift, h->d_xin, h->d_arena);
+        hipLaunchKernelGGL(k_blocks_rpy32, dim3(P.units), dim3(256), 0, s, h->d_blk, h->d_coord, h->CT, h->kp,
+                           h->d_shift, h->d_xin, h->d_arena);
+    else if (h->periodic)   // one-sided blocks
+        hipLaunchKernelGGL(k_blocks_rpy<true>, dim3(P.units), dim3(256), 0, s, h->d_blk, P.big, P.n, h->d_coord,
+                           h->CT, h->kp.p1, h->d_shift, h->d_xin, h->d_arena);
     else
-        hipLaunchKernelGGL((k_blocks_jit<KID, KD, double>), dim3(h->n_blk), dim3(256), 0, s, h->d_blk,
-                           h->d_coord, h->CT, h->kp, h->d_shift, h->d_xin, h->d_arena);
+        hipLaunchKernelGGL(k_blocks_rpy<false>, dim3(P.units), dim3(256), 0, s, h->d_blk, P.big, P.n, h->d_coord,
+                           h->CT, h->kp.p1, h->d_shift, h->d_xin, h->d_arena);
 }
 
 template <int KID, int KD>
@@ -284,7 +287,7 @@ static void dispatch_jit(h2p_hip_handle *h, hipStream_t s, int part) {
             else launch_jit2<KM, double>(h, s, part);
             break;
         default:
-            if (part == 0) launch_jit<KR, 3>(h, s);
+            if (part == 0) launch_rpy(h, s);
             break;
     }
 }
@@ -927,6 +930,46 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
         for (int i = 0; i < g->n_r_adm_pair; i++) adm_shift[i] = shift_index(g->per_adm_shifts + 3 * (size_t)i);
         for (int i = 0; i < g->n_r_inadm_pair; i++) inadm_shift[i] = shift_index(g->per_inadm_shifts + 3 * (size_t)i);
     }
+    // RPY: bounding box and largest radius of each node's points and of its
+    // skeleton points, from which a block knows that none of its pairs is
+    // within the sum of two radii (the tensor's far form; a margin of 1e-12
+    // covers the rounding of the kernel's own distances)
+    struct Extent { double lo[3], hi[3], a; };
+    std::vector<Extent> ext_pt, ext_sk;
+    const bool far_flags = krnl->id == KR && mode == H2P_HIP_JIT && prec == H2P_HIP_FP64;
+    if (far_flags) {
+        auto extent = [&](long long c, int n) {
+            Extent e;
+            for (int d = 0; d < 3; d++) e.lo[d] = HUGE_VAL, e.hi[d] = -HUGE_VAL;
+            e.a = 0.0;
+            for (int k = 0; k < n; k++) {
+                for (int d = 0; d < 3; d++) {
+                    const double v = cu[(size_t)d * CT + c + k];
+                    e.lo[d] = std::min(e.lo[d], v);
+                    e.hi[d] = std::max(e.hi[d], v);
+                }
+                e.a = std::max(e.a, cu[(size_t)3 * CT + c + k]);
+            }
+            return e;
+        };
+        ext_pt.resize(nn);
+        ext_sk.resize(nn);
+        for (int n = 0; n < nn; n++) {
+            if (g->pt_cluster[2 * n] < 0 || npt(n) < 0 || g->pt_cluster[2 * n + 1] >= g->n_point)
+                return bail(fail(H2P_HIP_EINVAL, "pt_cluster out of range"));
+            ext_pt[n] = extent(g->pt_cluster[2 * n], npt(n));
+            if (g->U_ncol[n] > 0) ext_sk[n] = extent(g->n_point + joff[n], g->J_npt[n]);
+        }
+    }
+    auto far_apart = [&](const Extent &a, const Extent &b, const double *shift) {
+        double d2 = 0.0;
+        for (int d = 0; d < 3; d++) {
+            const double s = shift ? shift[d] : 0.0;
+            const double gap = std::max({0.0, b.lo[d] + s - a.hi[d], a.lo[d] - (b.hi[d] + s)});
+            d2 += gap * gap;
+        }
+        return std::sqrt(d2) > (a.a + b.a) * (1.0 + 1e-12);   // false for NaN
+    };
     for (int i = 0; i < g->n_r_adm_pair; i++) {
         const int n0 = g->r_adm_pairs[2 * i], n1 = g->r_adm_pairs[2 * i + 1];
         const int l0 = g->node_level[n0], l1 = g->node_level[n1];
@@ -955,6 +998,9 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             t.out1 = arena; arena += t.ncol;
             (l0 > l1 ? dest_leaf[n1] : dest_y1[n1]).push_back(t.out1);
         }
+        if (far_flags && far_apart(l0 < l1 ? ext_pt[n0] : ext_sk[n0], l0 > l1 ? ext_pt[n1] : ext_sk[n1],
+                                   per ? g->per_adm_shifts + 3 * (size_t)i : nullptr))
+            t.flags |= H2P_BLK_FAR;
         B_pairs += (double)t.n0 * t.n1;
         blk.push_back(t);
         blk_deep.push_back(std::max(l0, l1) >= h->lv_cut ? 1 : 0);
@@ -994,6 +1040,9 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             t.flags = 0;
             t.out1 = -1;
         }
+        if (far_flags && i >= nlf &&
+            far_apart(ext_pt[n0], ext_pt[n1], per ? g->per_inadm_shifts + 3 * (size_t)(i - nlf) : nullptr))
+            t.flags |= H2P_BLK_FAR;
         D_pairs += (double)t.n0 * t.n1;
         if (t.nrow == 0 || t.ncol == 0) continue;
         blk.push_back(t);
@@ -1004,11 +1053,14 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
     // separately (the D blocks read only the permuted input, so they overlap
     // the sweeps); AOT and RPY handles keep one grouped launch.  Each part in
     // longest-processing-time order; the tiled kernels (FP64 Gaussian and
-    // Matern, FP32-mixed Coulomb, Gaussian and Matern) then run the small
+    // Matern, FP32-mixed Coulomb, Gaussian and Matern, FP64 RPY) then run the small
     // blocks of a part as wave units of four, after its workgroup-unit blocks.
     h->split = mode == H2P_HIP_JIT && h->kid != KR && !per;
-    const bool tiled = mode == H2P_HIP_JIT && h->kid != KR &&
-                       (prec == H2P_HIP_FP32MIX || h->kid == KG || h->kid == KM);
+    const bool tiled = mode == H2P_HIP_JIT && (h->kid == KR ? prec == H2P_HIP_FP64
+                                                            : prec == H2P_HIP_FP32MIX || h->kid == KG || h->kid == KM);
+    auto wave_task = [&](const BlkTask &t) {
+        return h->kid == KR ? rpy_wave_task(t.n0, t.n1) : jitm_wave_task(t.n0, t.n1);
+    };
     for (auto &P : h->part) P = h2p_hip_handle::BlkPart{};
     h->part[0].n = h->split ? nB_deep : h->n_blk;
     h->part[3].off = h->part[0].n;
@@ -1023,7 +1075,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
         });
         P.big = P.n;
         if (tiled)
-            P.big = (int)(std::stable_partition(b0, b1, [](const BlkTask &t) { return !jitm_wave_task(t.n0, t.n1); }) -
+            P.big = (int)(std::stable_partition(b0, b1, [&](const BlkTask &t) { return !wave_task(t); }) -
                           b0);
         P.units = P.big + (P.n - P.big + 3) / 4;
     }
@@ -2338,8 +2390,8 @@ static void launch_blocks_b(const BLaunch &b, const char *dbase, const ReqCtx *r
             else hipLaunchKernelGGL((k_blocks_jit2_b<KMW, double, 4>), grid, blk, 0, s, it, b.n_items, reqs);
             break;
         default:
-            if (f32) hipLaunchKernelGGL((k_blocks_jit_b<KR, 3, float>), grid, blk, 0, s, it, b.n_items, reqs);
-            else hipLaunchKernelGGL((k_blocks_jit_b<KR, 3, double>), grid, blk, 0, s, it, b.n_items, reqs);
+            if (f32) hipLaunchKernelGGL(k_blocks_rpy32_b, grid, blk, 0, s, it, b.n_items, reqs);
+            else hipLaunchKernelGGL(k_blocks_rpy_b, grid, blk, 0, s, it, b.n_items, reqs);
             break;
     }
 }

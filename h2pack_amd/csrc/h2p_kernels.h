@@ -22,7 +22,7 @@ struct BlkTask {
     int c0, c1;           // JIT: first point of each set in the unified coordinates
     int n0, n1;           // JIT: point counts
     int in0, in1;         // xin offsets of the operands (in0: ncol long, in1: nrow long)
-    int flags;            // bit 0: has out1
+    int flags;            // bit 0: has out1; bit 1 (RPY): no pair within two radii
     int shift;            // index into the shift table, added to set 1's coordinates
                           // (periodic images; entry 0 is the zero shift)
 };
@@ -452,6 +452,20 @@ __global__ void k_f64_to_f32(const double *__restrict__ in, float *__restrict__ 
     for (; i < n; i += stride) out[i] = (float)in[i];
 }
 
+// Orders the LDS accesses of one wave (LDS operations of a wave complete in
+// issue order; the fences keep the compiler from moving them).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int NW>
+__device__ __forceinline__ void jitm_sync() {
+    if constexpr (NW == 4) __syncthreads();
+    else wave_lds_sync();
+}
+
 // ---------------------------------------------------------------------------
 // Grouped kernel-evaluating bi-matvec for RPY (JIT), the krnl_bimv products
 // of src/H2Pack_matvec.c:586-764 (B) and :1002-1145 (D) with the 3x3 tensor
@@ -467,60 +481,46 @@ __global__ void k_f64_to_f32(const double *__restrict__ in, float *__restrict__ 
 #define H2P_JIT_ROWS 256                 // target rows staged per chunk (all JIT launches)
 #define H2P_JIT_MAXNS 4
 #define H2P_RPY_MAXNS 2
-// T = double: FP64.  T = float (FP32-mixed): coordinates relative to the
-// task's first target point (the differences taken in FP64, once per point,
-// then rounded), the tensor and the products in FP32; row sums leave the
-// pass as FP32 into the FP64 partials, column sums are FP32 over 16 rows
-// per lane and folded into FP64 registers.
-template <typename T>
-struct RpyRowT { T x, y, z, a, ia, v0, v1, v2; };
-using RpyRow = RpyRowT<double>;
+// FP32-mixed: coordinates relative to the task's first target point (the
+// differences taken in FP64, once per point, then rounded), the tensor and
+// the products in FP32; row sums leave the pass as FP32 into the FP64
+// partials, column sums are FP32 over 16 rows per lane and folded into FP64
+// registers.  (FP64: the tiled launch below.)
+struct RpyRow { float x, y, z, a, ia, v0, v1, v2; };
 
-template <int NS, typename T>
+template <int NS>
 __device__ __forceinline__ void rpy_pass(const BlkTask &t, int pbase, int npts,
                                          const double *__restrict__ cx, long long cstride, const KParam &kp,
                                          const double *__restrict__ shifts, const double *__restrict__ xin,
-                                         double *__restrict__ arena, RpyRowT<T> *rows,
+                                         double *__restrict__ arena, RpyRow *rows,
                                          double (*red)[3][4][H2P_WAVE], bool first) {
-    constexpr bool F32 = sizeof(T) == 4;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     // rows of cx: x, y, z, radius, reciprocal radius
     const double *cy = cx + cstride, *cz = cx + 2 * cstride, *ca = cx + 3 * cstride, *cia = cx + 4 * cstride;
     // set 1 may be a periodic image: its coordinates plus the task's shift
     double hx = shifts[3 * t.shift], hy = shifts[3 * t.shift + 1], hz = shifts[3 * t.shift + 2];
-    double ox = 0.0, oy = 0.0, oz = 0.0;
-    if constexpr (F32) {
-        ox = cx[t.c0];
-        oy = cy[t.c0];
-        oz = cz[t.c0];
-    }
-    T sx[NS], sy[NS], sz[NS], sa[NS], isa[NS], x0[NS][3], acc1[NS][3];
+    const double ox = cx[t.c0], oy = cy[t.c0], oz = cz[t.c0];
+    float sx[NS], sy[NS], sz[NS], sa[NS], isa[NS], x0[NS][3], acc1[NS][3];
     double acc1d[NS][3];
 #pragma unroll
     for (int k = 0; k < NS; k++) {
         const int p = k * H2P_WAVE + lane;
         const bool ok = p < npts;
         const int g = t.c1 + pbase + (ok ? p : 0);
-        if constexpr (F32) {
-            sx[k] = (T)(cx[g] + hx - ox);
-            sy[k] = (T)(cy[g] + hy - oy);
-            sz[k] = (T)(cz[g] + hz - oz);
-        } else {
-            sx[k] = cx[g] + hx;
-            sy[k] = cy[g] + hy;
-            sz[k] = cz[g] + hz;
-        }
-        sa[k] = (T)ca[g];
-        isa[k] = (T)cia[g];
+        sx[k] = (float)(cx[g] + hx - ox);
+        sy[k] = (float)(cy[g] + hy - oy);
+        sz[k] = (float)(cz[g] + hz - oz);
+        sa[k] = (float)ca[g];
+        isa[k] = (float)cia[g];
 #pragma unroll
         for (int b = 0; b < 3; b++) {
-            x0[k][b] = ok ? (T)xin[t.in0 + (pbase + p) * 3 + b] : (T)0;
-            acc1[k][b] = (T)0;
+            x0[k][b] = ok ? (float)xin[t.in0 + (pbase + p) * 3 + b] : 0.0f;
+            acc1[k][b] = 0.0f;
             acc1d[k][b] = 0.0;
         }
     }
     const bool has1 = t.flags & 1;
-    const T C = (T)kp.p1;
+    const float C = (float)kp.p1;
     int tile = 0;
     for (int rc = 0; rc < t.n0; rc += H2P_JIT_ROWS) {
         const int nr = min(t.n0 - rc, H2P_JIT_ROWS);
@@ -529,45 +529,39 @@ __device__ __forceinline__ void rpy_pass(const BlkTask &t, int pbase, int npts,
         for (int q = threadIdx.x; q < nr_pad; q += blockDim.x) {
             const bool ok = q < nr;
             const int g = t.c0 + rc + (ok ? q : 0);
-            RpyRowT<T> r;
-            if constexpr (F32) {
-                r.x = (T)(cx[g] - ox);
-                r.y = (T)(cy[g] - oy);
-                r.z = (T)(cz[g] - oz);
-            } else {
-                r.x = cx[g];
-                r.y = cy[g];
-                r.z = cz[g];
-            }
-            r.a = (T)ca[g];
-            r.ia = (T)cia[g];
+            RpyRow r;
+            r.x = (float)(cx[g] - ox);
+            r.y = (float)(cy[g] - oy);
+            r.z = (float)(cz[g] - oz);
+            r.a = (float)ca[g];
+            r.ia = (float)cia[g];
             const bool v = ok && has1;
-            r.v0 = v ? (T)xin[t.in1 + (rc + q) * 3] : (T)0;
-            r.v1 = v ? (T)xin[t.in1 + (rc + q) * 3 + 1] : (T)0;
-            r.v2 = v ? (T)xin[t.in1 + (rc + q) * 3 + 2] : (T)0;
+            r.v0 = v ? (float)xin[t.in1 + (rc + q) * 3] : 0.0f;
+            r.v1 = v ? (float)xin[t.in1 + (rc + q) * 3 + 1] : 0.0f;
+            r.v2 = v ? (float)xin[t.in1 + (rc + q) * 3 + 2] : 0.0f;
             rows[q] = r;
         }
         __syncthreads();
         for (int r0 = 4 * w; r0 < nr_pad; r0 += 16) {
-            T p[4][3];
+            float p[4][3];
             // one target at a time (the barriers bound the registers the
             // scheduler may spend on interleaving targets)
 #pragma unroll
             for (int a = 0; a < 4; a++) {
                 __builtin_amdgcn_sched_barrier(0);
-                const RpyRowT<T> R = rows[r0 + a];
-                p[a][0] = p[a][1] = p[a][2] = (T)0;
+                const RpyRow R = rows[r0 + a];
+                p[a][0] = p[a][1] = p[a][2] = 0.0f;
 #pragma unroll
                 for (int k = 0; k < NS; k++) {
                     const bool ok = (k * H2P_WAVE + lane) < npts;
-                    T t1, t2, ux, uy, uz;
+                    float t1, t2, ux, uy, uz;
                     rpy_coef_rcp(R.x - sx[k], R.y - sy[k], R.z - sz[k], R.a, sa[k], R.ia, isa[k], C,
                                  t1, t2, ux, uy, uz);
-                    t1 = ok ? t1 : (T)0;
-                    t2 = ok ? t2 : (T)0;
+                    t1 = ok ? t1 : 0.0f;
+                    t2 = ok ? t2 : 0.0f;
                     // K = t1 I + t2 u u^T (symmetric)
-                    const T ud0 = ux * x0[k][0] + uy * x0[k][1] + uz * x0[k][2];
-                    const T ud1 = ux * R.v0 + uy * R.v1 + uz * R.v2;
+                    const float ud0 = ux * x0[k][0] + uy * x0[k][1] + uz * x0[k][2];
+                    const float ud1 = ux * R.v0 + uy * R.v1 + uz * R.v2;
                     p[a][0] += t1 * x0[k][0] + t2 * ux * ud0;
                     p[a][1] += t1 * x0[k][1] + t2 * uy * ud0;
                     p[a][2] += t1 * x0[k][2] + t2 * uz * ud0;
@@ -580,24 +574,22 @@ __device__ __forceinline__ void rpy_pass(const BlkTask &t, int pbase, int npts,
             const int myrow = r0 + ((lane >> 4) & 3);
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                const T s = wave_sum4<T>(p[0][c], p[1][c], p[2][c], p[3][c]);
+                const float s = wave_sum4<float>(p[0][c], p[1][c], p[2][c], p[3][c]);
                 if ((lane & 15) == 0 && myrow < nr) {
                     double *o = arena + t.out0 + (rc + myrow) * 3 + c;
                     if (first) *o = (double)s;
                     else *o += (double)s;
                 }
             }
-            if constexpr (F32) {
-                if (++tile == 4) {
-                    tile = 0;
+            if (++tile == 4) {
+                tile = 0;
 #pragma unroll
-                    for (int k = 0; k < NS; k++)
+                for (int k = 0; k < NS; k++)
 #pragma unroll
-                        for (int b = 0; b < 3; b++) {
-                            acc1d[k][b] += (double)acc1[k][b];
-                            acc1[k][b] = (T)0;
-                        }
-                }
+                    for (int b = 0; b < 3; b++) {
+                        acc1d[k][b] += (double)acc1[k][b];
+                        acc1[k][b] = 0.0f;
+                    }
             }
         }
     }
@@ -607,8 +599,7 @@ __device__ __forceinline__ void rpy_pass(const BlkTask &t, int pbase, int npts,
         for (int k = 0; k < NS; k++)
 #pragma unroll
             for (int b = 0; b < 3; b++) {
-                if constexpr (F32) red[k][b][w][lane] = acc1d[k][b] + (double)acc1[k][b];
-                else red[k][b][w][lane] = acc1[k][b];
+                red[k][b][w][lane] = acc1d[k][b] + (double)acc1[k][b];
             }
         __syncthreads();
         for (int q = threadIdx.x; q < npts * 3; q += blockDim.x) {
@@ -620,32 +611,268 @@ __device__ __forceinline__ void rpy_pass(const BlkTask &t, int pbase, int npts,
     }
 }
 
-template <int KID, int KD, typename T = double>
-__device__ __forceinline__ void blocks_jit_body(const BlkTask &t, const double *__restrict__ cx,
-                                                long long cstride, const KParam &kp,
-                                                const double *__restrict__ shifts,
-                                                const double *__restrict__ xin,
+// FP64 RPY in tiles: a step covers 8 target x 16 source points, lane l the
+// pairs (4 k + l / 16, l % 16), k = 0, 1.
+//  * A pass covers up to 16 H2P_RPYT_NT source points, as evenly split over
+//    a block's passes as tiles allow (ranks of ~76 points are 5 tiles; lanes
+//    over 64 sources would leave 40% of them idle).  The points of both sets
+//    are staged in LDS, one array per component, so that a step reads its
+//    sources conflict-free and its targets by broadcast.
+//  * Row sums stay in the lane over the pass's tiles and are reduced over the
+//    16 lanes by DPP moves, column sums stay in registers over all rows.
+//  * The kernel is evaluated on the difference vector d itself, K = t1 I +
+//    g d d^T: no unit vector.  Blocks whose bounding boxes are further apart
+//    than two radii (flag H2P_BLK_FAR, set at upload) have only the far form,
+//      t1 = 1/r + (s / 3) / r^3,  g = (1 - s / r^2) / r^3,  s = a^2 + b^2,
+//    with 3 C / 4 folded into the staged inputs: 41 slots of the FP64 pipe
+//    per pair with both products, against 61 in the general form with its
+//    three regimes.
+//  * ONE (periodic handles): blocks act one way only.
+// Two launch units as in the norm-form kernels below: four waves share a
+// large block's rows, or take one small block each.
+// Bound by the FP64 pipe.  N = 20k at 20% volume fraction, us per launch: lanes
+// over 64 sources with the general form on every pair 796, this form 258;
+// periodic N = 10k: 1077 and 450.
+#define H2P_RPYT_NT 6
+#define H2P_RPYT_ROWS 64                      // targets staged per chunk (four workgroups' LDS fit a CU)
+#define H2P_RPYT_WAVE 96                      // a wave unit's most targets and sources
+#define H2P_RPYT_COMP 8                       // x y z a 1/a v0 v1 v2 (far: a^2 in place of a)
+#define H2P_RPYT_LDS (H2P_RPYT_COMP * (H2P_RPYT_ROWS + 16 * H2P_RPYT_NT))   // doubles per unit
+#define H2P_BLK_FAR 2
+
+// Whether an RPY task runs as a wave unit.
+__host__ __device__ inline bool rpy_wave_task(int n0, int n1) {
+    return n0 <= H2P_RPYT_WAVE && n1 <= 16 * H2P_RPYT_NT;
+}
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+    const long long b = __builtin_bit_cast(long long, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+
+// Sums over the 16 lanes of each lane group of two per-lane values; lanes
+// with bit 3 clear return the sum of v0, the others that of v1.  Row
+// rotation by 8, half-row mirror and quad permutations: VALU only.
+__device__ __forceinline__ double group16_sum2(double v0, double v1) {
+    const bool b3 = threadIdx.x & 8;
+    double a = (b3 ? v1 : v0) + dpp_move<0x128>(b3 ? v0 : v1);
+    a += dpp_move<0x141>(a);
+    a += dpp_move<0x4e>(a);
+    a += dpp_move<0xb1>(a);
+    return a;
+}
+
+// Stages points [0, n) of a set (padded with repeats and zero inputs to np).
+template <bool FAR>
+__device__ __forceinline__ void rpyt_stage(double *dst, int ld, int n, int np, int tid, int nthr, int c,
+                                           const double *__restrict__ cx, long long cstride, double hx, double hy,
+                                           double hz, const double *__restrict__ v, double vs) {
+    for (int q = tid; q < np; q += nthr) {
+        const bool ok = q < n;
+        const long long g = c + (ok ? q : 0);
+        const double a = cx[3 * cstride + g];
+        dst[q] = cx[g] + hx;
+        dst[ld + q] = cx[cstride + g] + hy;
+        dst[2 * ld + q] = cx[2 * cstride + g] + hz;
+        dst[3 * ld + q] = FAR ? a * a : a;
+        if (!FAR) dst[4 * ld + q] = cx[4 * cstride + g];
+#pragma unroll
+        for (int b = 0; b < 3; b++) dst[(5 + b) * ld + q] = (ok && v) ? v[3 * q + b] * vs : 0.0;
+    }
+}
+
+template <int NT, int NW, bool FAR, bool ONE>
+__device__ __forceinline__ void rpyt_pass(const BlkTask &t, int pbase, int npts, const double *__restrict__ cx,
+                                          long long cstride, double C, const double *__restrict__ shifts,
+                                          const double *__restrict__ xin, double *__restrict__ arena, double *lds,
+                                          double *red, bool first) {
+    constexpr int LR = H2P_RPYT_ROWS, LC = 16 * H2P_RPYT_NT;
+    const int lane = threadIdx.x & 63, w = NW == 4 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    const int tid = NW == 4 ? threadIdx.x : lane;
+    const int li = lane & 15, lg = lane >> 4;
+    double *rows = lds, *cols = lds + H2P_RPYT_COMP * LR;
+    const double vs = FAR ? 0.75 * C : 1.0;
+    const double *sh = shifts + 3 * t.shift;
+    const bool has1 = !ONE && (t.flags & 1);
+    rpyt_stage<FAR>(cols, LC, npts, 16 * NT, tid, NW * H2P_WAVE, t.c1 + pbase, cx, cstride, sh[0], sh[1], sh[2],
+                    xin + t.in0 + 3 * pbase, vs);
+    double acc[NT][3];
+#pragma unroll
+    for (int c = 0; c < NT; c++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) acc[c][b] = 0.0;
+    for (int rc = 0; rc < t.n0; rc += LR) {
+        const int nr = min(t.n0 - rc, LR);
+        const int nstep = (nr + 7) >> 3;
+        jitm_sync<NW>();
+        rpyt_stage<FAR>(rows, LR, nr, 8 * nstep, tid, NW * H2P_WAVE, t.c0 + rc, cx, cstride, 0.0, 0.0, 0.0,
+                        has1 ? xin + t.in1 + 3 * rc : nullptr, vs);
+        jitm_sync<NW>();
+        for (int st = w; st < nstep; st += NW) {
+            double r[2][8], p[2][3];
+            // an offset the compiler cannot see through: otherwise it keeps
+            // every tile's sources in registers across the steps and spills
+            int o0 = li;
+            asm volatile("" : "+v"(o0));
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    if (!(FAR && e == 4) && !(ONE && e >= 5)) r[k][e] = rows[e * LR + 8 * st + 4 * k + lg];
+                p[k][0] = p[k][1] = p[k][2] = 0.0;
+            }
+#pragma unroll
+            for (int c = 0; c < NT; c++) {
+                double s[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    if (!(FAR && e == 4)) s[e] = cols[e * LC + 16 * c + o0];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    double dx = r[k][0] - s[0], dy = r[k][1] - s[1], dz = r[k][2] - s[2], t1, g;
+                    if constexpr (FAR) {
+                        const double y = rsqrt_refined(__builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx)));
+                        const double y2 = y * y, sr = (r[k][3] + s[3]) * y2, y3 = y * y2;
+                        t1 = __builtin_fma(y * sr, 1.0 / 3.0, y);
+                        g = __builtin_fma(-sr, y3, y3);
+                    } else {
+                        double ux, uy, uz;
+                        rpy_coef_rcp(dx, dy, dz, r[k][3], s[3], r[k][4], s[4], C, t1, g, ux, uy, uz);
+                        dx = ux;
+                        dy = uy;
+                        dz = uz;
+                    }
+                    const double w0 = g * __builtin_fma(dz, s[7], __builtin_fma(dy, s[6], dx * s[5]));
+                    p[k][0] = __builtin_fma(w0, dx, __builtin_fma(t1, s[5], p[k][0]));
+                    p[k][1] = __builtin_fma(w0, dy, __builtin_fma(t1, s[6], p[k][1]));
+                    p[k][2] = __builtin_fma(w0, dz, __builtin_fma(t1, s[7], p[k][2]));
+                    if constexpr (!ONE) {
+                        const double w1 = g * __builtin_fma(dz, r[k][7], __builtin_fma(dy, r[k][6], dx * r[k][5]));
+                        acc[c][0] = __builtin_fma(w1, dx, __builtin_fma(t1, r[k][5], acc[c][0]));
+                        acc[c][1] = __builtin_fma(w1, dy, __builtin_fma(t1, r[k][6], acc[c][1]));
+                        acc[c][2] = __builtin_fma(w1, dz, __builtin_fma(t1, r[k][7], acc[c][2]));
+                        // pinned here: the compiler would sink the sums past the
+                        // row stores and keep every pair's t1, g and d alive
+                        asm volatile("" : "+v"(acc[c][0]), "+v"(acc[c][1]), "+v"(acc[c][2]));
+                    }
+                    asm volatile("" : "+v"(p[k][0]), "+v"(p[k][1]), "+v"(p[k][2]));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const int row = 8 * st + 4 * ((lane >> 3) & 1) + lg;
+#pragma unroll
+            for (int b = 0; b < 3; b++) {
+                const double v = group16_sum2(p[0][b], p[1][b]);
+                if ((lane & 7) == 0 && row < nr) {
+                    double *o = arena + t.out0 + 3 * (rc + row) + b;
+                    *o = first ? v : *o + v;
+                }
+            }
+        }
+    }
+    if (!has1) return;
+    // column sums: (g0 + g1) + (g2 + g3) over the lane groups, then the waves in order
+#pragma unroll
+    for (int c = 0; c < NT; c++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) {
+            double v = acc[c][b] + __shfl_xor(acc[c][b], 16, H2P_WAVE);
+            v += __shfl_xor(v, 32, H2P_WAVE);
+            const int j = 16 * c + li;
+            if constexpr (NW == 4) {
+                if (lg == 0) red[(w * 3 + b) * LC + j] = v;
+            } else {
+                if (lg == 0 && j < npts) arena[t.out1 + 3 * (pbase + j) + b] = v;
+            }
+        }
+    if constexpr (NW == 4) {
+        __syncthreads();
+        for (int q = threadIdx.x; q < 3 * npts; q += blockDim.x) {
+            const int j = q / 3, b = q - 3 * j;
+            arena[t.out1 + 3 * pbase + q] = (red[b * LC + j] + red[(3 + b) * LC + j]) +
+                                            (red[(6 + b) * LC + j] + red[(9 + b) * LC + j]);
+        }
+    }
+}
+
+template <int NW, bool FAR, bool ONE>
+__device__ __forceinline__ void rpyt_task(const BlkTask &t, const double *__restrict__ cx, long long cstride,
+                                          double C, const double *__restrict__ shifts,
+                                          const double *__restrict__ xin, double *__restrict__ arena, double *lds,
+                                          double *red) {
+    const int ntile = (t.n1 + 15) >> 4, npass = (ntile + H2P_RPYT_NT - 1) / H2P_RPYT_NT;
+    const int per = (ntile + npass - 1) / npass;   // tiles per pass, evenly
+    for (int c0 = 0; c0 < ntile; c0 += per) {
+        const int pb = 16 * c0, np = min(t.n1 - pb, 16 * per);
+        const bool first = c0 == 0;
+        switch ((np + 15) >> 4) {
+#define H2P_RPYT_CASE(n) \
+            case n: rpyt_pass<n, NW, FAR, ONE>(t, pb, np, cx, cstride, C, shifts, xin, arena, lds, red, first); break;
+            H2P_RPYT_CASE(1) H2P_RPYT_CASE(2) H2P_RPYT_CASE(3)
+            H2P_RPYT_CASE(4) H2P_RPYT_CASE(5) H2P_RPYT_CASE(6)
+#undef H2P_RPYT_CASE
+            default: break;
+        }
+        jitm_sync<NW>();
+    }
+}
+
+// Launch unit u: u < nbig runs task u on the whole workgroup, later units
+// tasks nbig + 4 (u - nbig) + w, one per wave.
+template <bool ONE>
+__device__ __forceinline__ void blocks_rpy_unit(const BlkTask *__restrict__ tasks, int u, int nbig, int ntask,
+                                                const double *__restrict__ cx, long long cstride, double C,
+                                                const double *__restrict__ shifts, const double *__restrict__ xin,
                                                 double *__restrict__ arena) {
-    static_assert(KID == KR && KD == 3, "the per-pass launch is the RPY kernel's");
-    __shared__ RpyRowT<T> rows[H2P_JIT_ROWS];
+    __shared__ double lds[4 * H2P_RPYT_LDS];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (u < nbig) {
+        const BlkTask t = tasks[u];
+        double *red = lds + H2P_RPYT_LDS;   // 4 x 3 x 16 NT doubles
+        if (t.flags & H2P_BLK_FAR) rpyt_task<4, true, ONE>(t, cx, cstride, C, shifts, xin, arena, lds, red);
+        else rpyt_task<4, false, ONE>(t, cx, cstride, C, shifts, xin, arena, lds, red);
+    } else {
+        const int i = nbig + 4 * (u - nbig) + w;
+        if (i >= ntask) return;
+        const BlkTask t = tasks[i];
+        double *l = lds + w * H2P_RPYT_LDS;
+        if (t.flags & H2P_BLK_FAR) rpyt_task<1, true, ONE>(t, cx, cstride, C, shifts, xin, arena, l, nullptr);
+        else rpyt_task<1, false, ONE>(t, cx, cstride, C, shifts, xin, arena, l, nullptr);
+    }
+}
+
+template <bool ONE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_blocks_rpy(const BlkTask *__restrict__ tasks, int nbig, int ntask, const double *__restrict__ cx,
+             long long cstride, double C, const double *__restrict__ shifts, const double *__restrict__ xin,
+             double *__restrict__ arena) {
+    blocks_rpy_unit<ONE>(tasks, blockIdx.x, nbig, ntask, cx, cstride, C, shifts, xin, arena);
+}
+
+// FP32-mixed RPY.
+__device__ __forceinline__ void blocks_rpy32(const BlkTask &t, const double *__restrict__ cx, long long cstride,
+                                             const KParam &kp, const double *__restrict__ shifts,
+                                             const double *__restrict__ xin, double *__restrict__ arena) {
+    __shared__ RpyRow rows[H2P_JIT_ROWS];
     __shared__ double red[H2P_RPY_MAXNS][3][4][H2P_WAVE];
     for (int pb = 0; pb < t.n1; pb += H2P_RPY_MAXNS * H2P_WAVE) {
         const int np = min(t.n1 - pb, H2P_RPY_MAXNS * H2P_WAVE);
         const bool first = (pb == 0);
-        if (np <= H2P_WAVE) rpy_pass<1, T>(t, pb, np, cx, cstride, kp, shifts, xin, arena, rows, red, first);
-        else rpy_pass<2, T>(t, pb, np, cx, cstride, kp, shifts, xin, arena, rows, red, first);
+        if (np <= H2P_WAVE) rpy_pass<1>(t, pb, np, cx, cstride, kp, shifts, xin, arena, rows, red, first);
+        else rpy_pass<2>(t, pb, np, cx, cstride, kp, shifts, xin, arena, rows, red, first);
         __syncthreads();
     }
 }
 
-template <int KID, int KD, typename T = double>
-__global__ void __launch_bounds__(256) k_blocks_jit(const BlkTask *__restrict__ tasks,
-                                                    const double *__restrict__ cx,
-                                                    long long cstride, KParam kp,
-                                                    const double *__restrict__ shifts,
-                                                    const double *__restrict__ xin,
-                                                    double *__restrict__ arena) {
-    blocks_jit_body<KID, KD, T>(tasks[blockIdx.x], cx, cstride, kp, shifts, xin, arena);
+__global__ void __launch_bounds__(256) k_blocks_rpy32(const BlkTask *__restrict__ tasks,
+                                                      const double *__restrict__ cx, long long cstride, KParam kp,
+                                                      const double *__restrict__ shifts,
+                                                      const double *__restrict__ xin, double *__restrict__ arena) {
+    blocks_rpy32(tasks[blockIdx.x], cx, cstride, kp, shifts, xin, arena);
 }
 
 // The root's periodic block (H2P_matvec_periodic, src/H2Pack_matvec_periodic.c:
@@ -815,20 +1042,6 @@ struct JitmNV { double n, v; };    // |r|^2 and the transposed product's input
 #define H2P_JITM_LDS_WG (6 * H2P_JIT_ROWS + 5 * 16 * H2P_JITM_NT + 4 * H2P_JITM_NT * H2P_WAVE)
 #define H2P_JITM_LDS_WAVE (6 * H2P_JITW_ROWS + 5 * 16 * H2P_JITM_NT)
 #define H2P_JITM_LDS (H2P_JITM_LDS_WG > 4 * H2P_JITM_LDS_WAVE ? H2P_JITM_LDS_WG : 4 * H2P_JITM_LDS_WAVE)
-
-// Orders the LDS accesses of one wave (LDS operations of a wave complete in
-// issue order; the fences keep the compiler from moving them).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-template <int NW>
-__device__ __forceinline__ void jitm_sync() {
-    if constexpr (NW == 4) __syncthreads();
-    else wave_lds_sync();
-}
 
 template <int KID, int NT, int NW>
 __device__ __forceinline__ void jitm_pass(const BlkTask &t, int pbase, int npts,
