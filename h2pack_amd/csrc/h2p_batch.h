@@ -73,7 +73,7 @@ __global__ void __launch_bounds__(256) k_fwd2_b(const BatchItem *__restrict__ it
 }
 
 // WPE: waves per SIMD the kernel is compiled for (1: no constraint); the
-// tiled kernels run at 4, as the single-matrix launch's occupancy variant.
+// tiled kernels run at 4, as the single-matrix launch's default.
 template <int KID, typename T, int WPE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
 k_blocks_jit2_b(const BatchItem *__restrict__ items, int n, const ReqCtx *__restrict__ reqs) {

@@ -930,13 +930,14 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
         for (int i = 0; i < g->n_r_adm_pair; i++) adm_shift[i] = shift_index(g->per_adm_shifts + 3 * (size_t)i);
         for (int i = 0; i < g->n_r_inadm_pair; i++) inadm_shift[i] = shift_index(g->per_inadm_shifts + 3 * (size_t)i);
     }
-    // RPY: bounding box and largest radius of each node's points and of its
-    // skeleton points, from which a block knows that none of its pairs is
-    // within the sum of two radii (the tensor's far form; a margin of 1e-12
-    // covers the rounding of the kernel's own distances)
+    // FP64 RPY and Coulomb: bounding box and largest radius (Coulomb: 0) of
+    // each node's points and of its skeleton points, from which a block knows
+    // that none of its pairs is within the sum of two radii, or coincident
+    // (a margin of 1e-12 covers the rounding of the kernel's own distances,
+    // and gaps below 1e-100 could still have a distance whose square is 0)
     struct Extent { double lo[3], hi[3], a; };
     std::vector<Extent> ext_pt, ext_sk;
-    const bool far_flags = krnl->id == KR && mode == H2P_HIP_JIT && prec == H2P_HIP_FP64;
+    const bool far_flags = (krnl->id == KR || krnl->id == KC) && mode == H2P_HIP_JIT && prec == H2P_HIP_FP64;
     if (far_flags) {
         auto extent = [&](long long c, int n) {
             Extent e;
@@ -948,7 +949,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
                     e.lo[d] = std::min(e.lo[d], v);
                     e.hi[d] = std::max(e.hi[d], v);
                 }
-                e.a = std::max(e.a, cu[(size_t)3 * CT + c + k]);
+                if (xd > 3) e.a = std::max(e.a, cu[(size_t)3 * CT + c + k]);
             }
             return e;
         };
@@ -968,7 +969,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             const double gap = std::max({0.0, b.lo[d] + s - a.hi[d], a.lo[d] - (b.hi[d] + s)});
             d2 += gap * gap;
         }
-        return std::sqrt(d2) > (a.a + b.a) * (1.0 + 1e-12);   // false for NaN
+        return std::sqrt(d2) > std::max((a.a + b.a) * (1.0 + 1e-12), 1e-100);   // false for NaN
     };
     for (int i = 0; i < g->n_r_adm_pair; i++) {
         const int n0 = g->r_adm_pairs[2 * i], n1 = g->r_adm_pairs[2 * i + 1];
@@ -1052,12 +1053,11 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
     // JIT handles of the scalar kernels launch the B blocks and the D blocks
     // separately (the D blocks read only the permuted input, so they overlap
     // the sweeps); AOT and RPY handles keep one grouped launch.  Each part in
-    // longest-processing-time order; the tiled kernels (FP64 Gaussian and
-    // Matern, FP32-mixed Coulomb, Gaussian and Matern, FP64 RPY) then run the small
-    // blocks of a part as wave units of four, after its workgroup-unit blocks.
+    // longest-processing-time order; the tiled kernels (all but FP32-mixed
+    // RPY) then run the small blocks of a part as wave units of four, after
+    // its workgroup-unit blocks.
     h->split = mode == H2P_HIP_JIT && h->kid != KR && !per;
-    const bool tiled = mode == H2P_HIP_JIT && (h->kid == KR ? prec == H2P_HIP_FP64
-                                                            : prec == H2P_HIP_FP32MIX || h->kid == KG || h->kid == KM);
+    const bool tiled = mode == H2P_HIP_JIT && !(h->kid == KR && prec == H2P_HIP_FP32MIX);
     auto wave_task = [&](const BlkTask &t) {
         return h->kid == KR ? rpy_wave_task(t.n0, t.n1) : jitm_wave_task(t.n0, t.n1);
     };
@@ -2379,7 +2379,7 @@ static void launch_blocks_b(const BLaunch &b, const char *dbase, const ReqCtx *r
     switch (b.kid) {
         case KC:
             if (f32) hipLaunchKernelGGL((k_blocks_jit2_b<KC, float, 4>), grid, blk, 0, s, it, b.n_items, reqs);
-            else hipLaunchKernelGGL((k_blocks_jit2_b<KC, double, 1>), grid, blk, 0, s, it, b.n_items, reqs);
+            else hipLaunchKernelGGL((k_blocks_jit2_b<KC, double, 4>), grid, blk, 0, s, it, b.n_items, reqs);
             break;
         case KG:
             if (f32) hipLaunchKernelGGL((k_blocks_jit2_b<KG, float, 4>), grid, blk, 0, s, it, b.n_items, reqs);

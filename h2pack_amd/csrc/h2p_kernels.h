@@ -22,10 +22,14 @@ struct BlkTask {
     int c0, c1;           // JIT: first point of each set in the unified coordinates
     int n0, n1;           // JIT: point counts
     int in0, in1;         // xin offsets of the operands (in0: ncol long, in1: nrow long)
-    int flags;            // bit 0: has out1; bit 1 (RPY): no pair within two radii
+    int flags;            // bit 0: has out1; bit 1 (H2P_BLK_FAR): the boxes of the two sets are apart
     int shift;            // index into the shift table, added to set 1's coordinates
                           // (periodic images; entry 0 is the zero shift)
 };
+
+// The two point sets' bounding boxes are apart: no coincident pair, and for
+// RPY no pair within the sum of two radii.
+#define H2P_BLK_FAR 2
 
 // Upward-sweep task: y0[out] = U^T in, U row-major nrow x r.
 #define H2P_FWD_MIN_WG 256    // a level's upward tasks narrow their column chunks to reach this many (one per CU)
@@ -479,7 +483,6 @@ __device__ __forceinline__ void jitm_sync() {
 //    butterflies (one per component).
 //  * Lanes without a source point use a valid point with zero coefficients.
 #define H2P_JIT_ROWS 256                 // target rows staged per chunk (all JIT launches)
-#define H2P_JIT_MAXNS 4
 #define H2P_RPY_MAXNS 2
 // FP32-mixed: coordinates relative to the task's first target point (the
 // differences taken in FP64, once per point, then rounded), the tensor and
@@ -638,7 +641,6 @@ __device__ __forceinline__ void rpy_pass(const BlkTask &t, int pbase, int npts,
 #define H2P_RPYT_WAVE 96                      // a wave unit's most targets and sources
 #define H2P_RPYT_COMP 8                       // x y z a 1/a v0 v1 v2 (far: a^2 in place of a)
 #define H2P_RPYT_LDS (H2P_RPYT_COMP * (H2P_RPYT_ROWS + 16 * H2P_RPYT_NT))   // doubles per unit
-#define H2P_BLK_FAR 2
 
 // Whether an RPY task runs as a wave unit.
 __host__ __device__ inline bool rpy_wave_task(int n0, int n1) {
@@ -891,108 +893,6 @@ __global__ void __launch_bounds__(256) k_root_block(const double *__restrict__ p
 }
 
 // ---------------------------------------------------------------------------
-// Grouped kernel-evaluating bi-matvec for FP64 Coulomb.  1/r has the
-// kernel's diagonal value at r = 0, so r = 0 must be exact: the distances
-// are formed from coordinate differences.
-//  * Source points (columns) live in lanes, NS strips of 64 per pass.
-//  * Target points (rows) are staged in LDS; each wave takes four rows per
-//    iteration and reduces the four row sums with one butterfly.
-//  * Lanes without a source point use a valid point with x = 0, so every
-//    kernel value stays finite and no per-pair select is needed.
-struct JitRow { double x, y, z, v; };    // coordinates and the transposed product's input
-
-template <int NS>
-__device__ __forceinline__ void jitc_pass(const BlkTask &t, int pbase, int npts,
-                                          const double *__restrict__ cx, long long cstride, double diag,
-                                          const double *__restrict__ xin, double *__restrict__ arena,
-                                          JitRow *rows, double (*red)[4][H2P_WAVE], bool first) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const double *cy = cx + cstride, *cz = cx + 2 * cstride;
-    double sx[NS], sy[NS], sz[NS], x0[NS], acc1[NS];
-#pragma unroll
-    for (int k = 0; k < NS; k++) {
-        const int p = k * H2P_WAVE + lane;
-        const bool ok = p < npts;
-        const int g = t.c1 + pbase + (ok ? p : 0);
-        sx[k] = cx[g];
-        sy[k] = cy[g];
-        sz[k] = cz[g];
-        x0[k] = ok ? xin[t.in0 + pbase + p] : 0.0;
-        acc1[k] = 0.0;
-    }
-    const bool has1 = t.flags & 1;
-    for (int rc = 0; rc < t.n0; rc += H2P_JIT_ROWS) {
-        const int nr = min(t.n0 - rc, H2P_JIT_ROWS);
-        const int nr_pad = (nr + 15) & ~15;
-        __syncthreads();
-        for (int q = threadIdx.x; q < nr_pad; q += blockDim.x) {
-            const bool ok = q < nr;
-            const int g = t.c0 + rc + (ok ? q : 0);
-            JitRow r;
-            r.x = cx[g];
-            r.y = cy[g];
-            r.z = cz[g];
-            r.v = (ok && has1) ? xin[t.in1 + rc + q] : 0.0;
-            rows[q] = r;
-        }
-        __syncthreads();
-        for (int r0 = 4 * w; r0 < nr_pad; r0 += 16) {
-            double p[4];
-            JitRow rr[4];
-#pragma unroll
-            for (int a = 0; a < 4; a++) {
-                rr[a] = rows[r0 + a];
-                p[a] = 0.0;
-            }
-#pragma unroll
-            for (int k = 0; k < NS; k++) {
-#pragma unroll
-                for (int a = 0; a < 4; a++) {
-                    const double dx = rr[a].x - sx[k], dy = rr[a].y - sy[k], dz = rr[a].z - sz[k];
-                    const double kv = kprep<KC>(dx * dx + dy * dy + dz * dz, diag);
-                    p[a] += kv * x0[k];
-                    acc1[k] += kv * rr[a].v;
-                }
-            }
-            const double s = wave_sum4<double>(p[0], p[1], p[2], p[3]);
-            const int myrow = r0 + ((lane >> 4) & 3);
-            if ((lane & 15) == 0 && myrow < nr) {
-                double *o = arena + t.out0 + rc + myrow;
-                if (first) *o = s;
-                else *o += s;
-            }
-        }
-    }
-    if (has1) {
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < NS; k++) red[k][w][lane] = acc1[k];
-        __syncthreads();
-        for (int c = threadIdx.x; c < npts; c += blockDim.x) {
-            const int k = c >> 6, l = c & 63;
-            arena[t.out1 + pbase + c] = (red[k][0][l] + red[k][1][l]) + (red[k][2][l] + red[k][3][l]);
-        }
-    }
-}
-
-__device__ __forceinline__ void blocks_jitc(const BlkTask &t, const double *__restrict__ cx, long long cstride,
-                                            double diag, const double *__restrict__ xin,
-                                            double *__restrict__ arena) {
-    __shared__ JitRow rows[H2P_JIT_ROWS];
-    __shared__ double red[H2P_JIT_MAXNS][4][H2P_WAVE];
-    for (int pb = 0; pb < t.n1; pb += H2P_JIT_MAXNS * H2P_WAVE) {
-        const int np = min(t.n1 - pb, H2P_JIT_MAXNS * H2P_WAVE);
-        const int ns = (np + 63) >> 6;
-        const bool first = (pb == 0);
-        if (ns <= 1) jitc_pass<1>(t, pb, np, cx, cstride, diag, xin, arena, rows, red, first);
-        else if (ns <= 2) jitc_pass<2>(t, pb, np, cx, cstride, diag, xin, arena, rows, red, first);
-        else if (ns <= 3) jitc_pass<3>(t, pb, np, cx, cstride, diag, xin, arena, rows, red, first);
-        else jitc_pass<4>(t, pb, np, cx, cstride, diag, xin, arena, rows, red, first);
-        __syncthreads();
-    }
-}
-
-// ---------------------------------------------------------------------------
 // FP64 norm-form kernels (Gaussian, Matern) with the distances on the matrix
 // cores.  The squared distances of a tile of 16 target rows x 16 source
 // columns are one v_mfma_f64_16x16x4f64,
@@ -1208,6 +1108,160 @@ __device__ __forceinline__ void blocks_jitm_unit(const BlkTask *__restrict__ tas
 }
 
 // ---------------------------------------------------------------------------
+// FP64 Coulomb in the same tiling and launch units, with the distances from
+// coordinate differences on the VALU: 1/r has the kernel's diagonal value at
+// r = 0, so r = 0 must be exact.
+//  * A pass's sources are staged in LDS, one array per component; a lane
+//    reads its column's point once per tile for its four rows, whose
+//    coordinates stay in registers.
+//  * Blocks whose bounding boxes are apart (H2P_BLK_FAR) have no coincident
+//    pair and skip the test for one (3 of 19 slots per pair).
+// Bound by the FP64 pipe.  N = 200k, density 10 (1.4e9 pairs): B launches 2127
+// us with sources in 64-lane strips (ranks of ~80 points leave a third of them
+// idle), 1223 us in tiles; D launches 272 and 135.
+#define H2P_JITC_LDS_WG (4 * H2P_JIT_ROWS + 4 * 16 * H2P_JITM_NT + 4 * 16 * H2P_JITM_NT)
+#define H2P_JITC_LDS_WAVE (4 * H2P_JITW_ROWS + 4 * 16 * H2P_JITM_NT)
+#define H2P_JITC_LDS (H2P_JITC_LDS_WG > 4 * H2P_JITC_LDS_WAVE ? H2P_JITC_LDS_WG : 4 * H2P_JITC_LDS_WAVE)
+
+template <int NT, int NW, bool FAR>
+__device__ __forceinline__ void jitc_pass(const BlkTask &t, int pbase, int npts, const double *__restrict__ cx,
+                                          long long cstride, double diag, const double *__restrict__ xin,
+                                          double *__restrict__ arena, double *rows, double *cols, double *red,
+                                          bool first) {
+    constexpr int ROWS = NW == 4 ? H2P_JIT_ROWS : H2P_JITW_ROWS, LC = 16 * H2P_JITM_NT;
+    const int lane = threadIdx.x & 63, w = NW == 4 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    const int tid = NW == 4 ? threadIdx.x : lane;
+    const int li = lane & 15, lg = lane >> 4;
+    const bool has1 = t.flags & 1;
+    // one set in LDS: x, y, z, input value (padding repeats a point, input 0)
+    auto stage = [&](double *dst, int ld, int n, int np, int c, const double *v) {
+        for (int q = tid; q < np; q += NW * H2P_WAVE) {
+            const bool ok = q < n;
+            const long long g = c + (ok ? q : 0);
+            dst[q] = cx[g];
+            dst[ld + q] = cx[cstride + g];
+            dst[2 * ld + q] = cx[2 * cstride + g];
+            dst[3 * ld + q] = (ok && v) ? v[q] : 0.0;
+        }
+    };
+    stage(cols, LC, npts, 16 * NT, t.c1 + pbase, xin + t.in0 + pbase);
+    double acc[NT];
+#pragma unroll
+    for (int c = 0; c < NT; c++) acc[c] = 0.0;
+    for (int rc = 0; rc < t.n0; rc += ROWS) {
+        const int nr = min(t.n0 - rc, ROWS);
+        const int ntile = (nr + 15) >> 4;
+        jitm_sync<NW>();
+        stage(rows, ROWS, nr, 16 * ntile, t.c0 + rc, has1 ? xin + t.in1 + rc : nullptr);
+        jitm_sync<NW>();
+        for (int tt = w; tt < ntile; tt += NW) {
+            double rx[4], ry[4], rz[4], rv[4], p[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int q = tt * 16 + 4 * r + lg;
+                rx[r] = rows[q];
+                ry[r] = rows[ROWS + q];
+                rz[r] = rows[2 * ROWS + q];
+                rv[r] = rows[3 * ROWS + q];
+                p[r] = 0.0;
+            }
+            // an offset the compiler cannot see through, or it keeps every
+            // tile's sources in registers across the row tiles
+            int o = li;
+            asm volatile("" : "+v"(o));
+            auto tile = [&](auto nrq) {
+                constexpr int NR = decltype(nrq)::value;
+#pragma unroll
+                for (int c = 0; c < NT; c++) {
+                    const double sx = cols[16 * c + o], sy = cols[LC + 16 * c + o], sz = cols[2 * LC + 16 * c + o],
+                                 sv = cols[3 * LC + 16 * c + o];
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int r = 0; r < NR; r++) {
+                        const double dx = rx[r] - sx, dy = ry[r] - sy, dz = rz[r] - sz;
+                        const double q = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+                        double kv = rsqrt_refined(q);   // NaN at q = 0, replaced
+                        if constexpr (!FAR) kv = q == 0.0 ? diag : kv;
+                        p[r] = __builtin_fma(kv, sv, p[r]);
+                        acc[c] = __builtin_fma(kv, rv[r], acc[c]);
+                        asm volatile("" : "+v"(acc[c]));   // not sunk past the row stores
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            tile_rows(nr - tt * 16, tile);
+            const double s = group16_sum4(p[0], p[1], p[2], p[3]);
+            const int myrow = tt * 16 + 4 * ((lane >> 2) & 3) + lg;
+            if ((lane & 3) == 0 && myrow < nr) {
+                double *o2 = arena + t.out0 + rc + myrow;
+                if (first) *o2 = s;
+                else *o2 += s;
+            }
+        }
+    }
+    if (!has1) return;
+    // (g0 + g1) + (g2 + g3) over the lane groups, then the waves in order
+#pragma unroll
+    for (int c = 0; c < NT; c++) {
+        double s = acc[c] + __shfl_xor(acc[c], 16, H2P_WAVE);
+        s += __shfl_xor(s, 32, H2P_WAVE);
+        const int j = 16 * c + li;
+        if constexpr (NW == 4) {
+            if (lg == 0) red[w * LC + j] = s;
+        } else {
+            if (lg == 0 && j < npts) arena[t.out1 + pbase + j] = s;
+        }
+    }
+    if constexpr (NW == 4) {
+        __syncthreads();
+        for (int j = threadIdx.x; j < npts; j += blockDim.x)
+            arena[t.out1 + pbase + j] = (red[j] + red[LC + j]) + (red[2 * LC + j] + red[3 * LC + j]);
+    }
+}
+
+template <int NW, bool FAR>
+__device__ __forceinline__ void jitc_task(const BlkTask &t, const double *__restrict__ cx, long long cstride,
+                                          double diag, const double *__restrict__ xin, double *__restrict__ arena,
+                                          double *lds) {
+    constexpr int ROWS = NW == 4 ? H2P_JIT_ROWS : H2P_JITW_ROWS;
+    double *cols = lds + 4 * ROWS, *red = cols + 4 * 16 * H2P_JITM_NT;   // red: workgroup unit only
+    const int ntile = (t.n1 + 15) >> 4, npass = (ntile + H2P_JITM_NT - 1) / H2P_JITM_NT;
+    const int per = npass > 0 ? (ntile + npass - 1) / npass : 1;   // tiles per pass, evenly
+    for (int c0 = 0; c0 < ntile; c0 += per) {
+        const int pb = 16 * c0, np = min(t.n1 - pb, 16 * per);
+        const bool first = c0 == 0;
+        switch ((np + 15) >> 4) {
+#define H2P_JITC_CASE(n) \
+            case n: jitc_pass<n, NW, FAR>(t, pb, np, cx, cstride, diag, xin, arena, lds, cols, red, first); break;
+            H2P_JITC_CASE(1) H2P_JITC_CASE(2) H2P_JITC_CASE(3) H2P_JITC_CASE(4)
+            H2P_JITC_CASE(5) H2P_JITC_CASE(6) H2P_JITC_CASE(7) H2P_JITC_CASE(8)
+#undef H2P_JITC_CASE
+            default: break;
+        }
+        jitm_sync<NW>();
+    }
+}
+
+__device__ __forceinline__ void blocks_jitc_unit(const BlkTask *__restrict__ tasks, int u, int nbig, int ntask,
+                                                 const double *__restrict__ cx, long long cstride, double diag,
+                                                 const double *__restrict__ xin, double *__restrict__ arena) {
+    __shared__ double lds[H2P_JITC_LDS];
+    if (u < nbig) {
+        const BlkTask t = tasks[u];
+        if (t.flags & H2P_BLK_FAR) jitc_task<4, true>(t, cx, cstride, diag, xin, arena, lds);
+        else jitc_task<4, false>(t, cx, cstride, diag, xin, arena, lds);
+    } else {
+        const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int i = nbig + 4 * (u - nbig) + w;
+        if (i >= ntask) return;
+        const BlkTask t = tasks[i];
+        double *l = lds + w * H2P_JITC_LDS_WAVE;
+        if (t.flags & H2P_BLK_FAR) jitc_task<1, true>(t, cx, cstride, diag, xin, arena, l);
+        else jitc_task<1, false>(t, cx, cstride, diag, xin, arena, l);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // FP32-mixed scalar kernels (Coulomb, Gaussian, Matern) in the same tiling
 // and launch units, with the distances on the VALU from coordinate
 // differences (FP32 keeps differences for accuracy, and Coulomb's r = 0 stays
@@ -1394,9 +1448,7 @@ __host__ __device__ inline bool jitm_wave_task(int n0, int n1) {
     return n0 <= H2P_JITW_ROWS && n1 <= 16 * H2P_JITM_NT;
 }
 
-// Launch unit u of the grouped kernel-evaluating launch: the FP64 norm-form
-// kernels and the FP32-mixed kernels run workgroup and wave units, FP64
-// Coulomb one task per workgroup (nbig = ntask).
+// Launch unit u of the grouped kernel-evaluating launch.
 template <int KID, typename T>
 __device__ __forceinline__ void blocks_jit2_unit(const BlkTask *__restrict__ tasks, int u, int nbig, int ntask,
                                                  const double *__restrict__ cx, long long cstride,
@@ -1408,7 +1460,7 @@ __device__ __forceinline__ void blocks_jit2_unit(const BlkTask *__restrict__ tas
         blocks_jitm_unit<KID>(tasks, u, nbig, ntask, cx, cstride, scale, diag, xin, arena);
     } else {
         static_assert(KID == KC, "scalar kernels only");
-        blocks_jitc(tasks[u], cx, cstride, diag, xin, arena);
+        blocks_jitc_unit(tasks, u, nbig, ntask, cx, cstride, diag, xin, arena);
     }
 }
 
