@@ -18,15 +18,10 @@ namespace h2p {
 typedef double d4 __attribute__((ext_vector_type(4)));   // one lane's share of a 16x16 FP64 MFMA tile
 typedef float f4 __attribute__((ext_vector_type(4)));    // one lane's share of a 16x16 FP32 MFMA tile
 
-// Kernel ids.  KGW / KMW are Gaussian / Matern-3/2 for FP64 JIT handles
-// whose point extent can push the exponential's argument past the range of
-// the unclamped exp2_neg: their kernel values clamp the argument first
-// (bitwise the same values wherever the unclamped form is in range).
-enum { KC = 0, KG = 1, KM = 2, KR = 3, KGW = 4, KMW = 5 };
+// Kernel ids (Coulomb, Gaussian, Matern-3/2, RPY).
+enum { KC = 0, KG = 1, KM = 2, KR = 3 };
 
-__host__ __device__ constexpr int kbase(int kid) { return kid == KGW ? KG : kid == KMW ? KM : kid; }
-
-// the table of exp2_neg, copied into LDS by the kernels that use it
+// the table of the exponentials, copied into LDS by the kernels that use it
 __constant__ double c_e2tab[H2P_E2_N] = {H2P_E2_TABLE};
 
 struct KParam {
@@ -167,6 +162,21 @@ __device__ __forceinline__ double rsqrt_refined(double q) {
     return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
 }
 
+// sqrt(q) of a squared distance in FP64.  q below 1e-300 (0, or rounded
+// negative by the norm-expanded distance) counts as about 1e-300, by one
+// integer maximum on the upper word.  With y the estimate of 1/sqrt(q) and
+// g = q y, e = 1 - g y: sqrt(q) = g (1 + e (1/2 + 3/8 e)) to third order, one
+// operation less than q times the refined reciprocal root.
+__device__ __forceinline__ double sqrt_floored(double q) {
+    const long long b = __builtin_bit_cast(long long, q);
+    const int hi = (int)(b >> 32), fl = 0x01a56e1f;   // upper word of 1e-300
+    q = __builtin_bit_cast(double, ((long long)(hi > fl ? hi : fl) << 32) | (unsigned)b);
+    const double y = __builtin_amdgcn_rsq(q);
+    const double g = q * y;
+    const double e = __builtin_fma(-g, y, 1.0);
+    return __builtin_fma(g * e, __builtin_fma(0.375, e, 0.5), g);
+}
+
 // Scalar kernels on prepared squared distances.  Coordinates are scaled
 // before the distance is formed so that the kernels need no parameter:
 //   Gaussian exp(-l r^2)          : scale sqrt(128 l log2 e) -> K = 2^(-q / 128)
@@ -181,18 +191,33 @@ __device__ __forceinline__ double kprep(double q, double diag, const double *e2t
         const double y = rsqrt_refined(z ? 1.0 : q);   // branch-free
         return z ? diag : y;
     } else if constexpr (KID == KG) {
-        return exp2_neg128(q, e2t);
-    } else if constexpr (KID == KGW) {
         return exp2_neg128_clamped(q, e2t);
     } else {
-        static_assert(KID == KM || KID == KMW, "scalar kernels only");
-        // sqrt(q) as q / sqrt(q); the clamp keeps q = 0 (and a rounded
-        // negative q from the norm-expanded distance) finite, s ~ 1e-150
-        const double qq = __builtin_fmax(q, 1e-300);
-        const double s = qq * rsqrt_refined(qq);
+        static_assert(KID == KM, "scalar kernels only");
+        const double s = sqrt_floored(q);
         const double x = s * (128.0 * 1.4426950408889634);   // e^(-s) = 2^(-x / 128)
-        const double e = KID == KM ? exp2_neg128(x, e2t) : exp2_neg128_clamped(x, e2t);
+        const double e = exp2_neg128_clamped(x, e2t);
         return __builtin_fma(s, e, e);
+    }
+}
+
+// The same for the matvec's norm-form launches, NR values at once (so that NR
+// table reads are in flight); FAST as for exp2_neg128x.
+template <int KID, bool FAST, int NR>
+__device__ __forceinline__ void kjit(const d4 &q, const double *e2x, double c2, double *kv) {
+    static_assert(KID == KG || KID == KM, "norm-form kernels only");
+    E2X e[NR];
+    double s[NR];
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        s[r] = KID == KM ? sqrt_floored(q[r]) : 0.0;
+        e[r] = exp2_neg128x_begin<FAST>(KID == KM ? s[r] * (128.0 * 1.4426950408889634) : q[r], e2x);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        kv[r] = exp2_neg128x_end<FAST>(e[r], c2);
+        if constexpr (KID == KM) kv[r] = __builtin_fma(s[r], kv[r], kv[r]);
     }
 }
 
@@ -212,8 +237,8 @@ __device__ __forceinline__ float kprep(float q, float diag) {
 // Coordinate scale of the prepared forms: the FP64 kernels above (f64) and
 // the FP32 ones (Gaussian K = 2^(-q) there).
 __host__ __device__ inline double kscale(int kid, double p0, bool f64) {
-    if (kbase(kid) == KG) return __builtin_sqrt(p0 * 1.4426950408889634 * (f64 ? 128.0 : 1.0));
-    if (kbase(kid) == KM) return 1.7320508075688772 * p0;
+    if (kid == KG) return __builtin_sqrt(p0 * 1.4426950408889634 * (f64 ? 128.0 : 1.0));
+    if (kid == KM) return 1.7320508075688772 * p0;
     return 1.0;
 }
 

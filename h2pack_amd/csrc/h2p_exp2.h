@@ -2,7 +2,7 @@
 // method: P. T. P. Tang, "Table-driven implementation of the exponential
 // function in IEEE floating-point arithmetic", ACM TOMS 15(2), 1989, here in
 // base 2 with 128 table entries).  Used by the FP64 Gaussian and Matern-3/2
-// kernel evaluations of the JIT block launches, whose arguments arrive
+// kernel evaluations of the matmul, whose arguments arrive
 // already multiplied by 128 (the Gaussian through its coordinate scale);
 // the reference evaluates the same kernels through its SIMD library's exp
 // (src/H2Pack_3D_kernels.h:212-268, 433-497).
@@ -100,6 +100,71 @@ H2P_HD inline double exp2_neg128_clamped(double x, const double *tab) {
     b = ((uint64_t)(uint32_t)(hi < cl ? hi : cl) << 32) | (uint32_t)b;
     __builtin_memcpy(&x, &b, sizeof b);
     return exp2_neg128(x, tab);
+}
+
+// ---------------------------------------------------------------------------
+// The same exponential for the matvec's kernel values, on a table whose upper
+// words are stored minus their index << 13 (e2x_entry): adding the rounded
+// argument << 13 gives 2^floor(k / 128) * 2^((k mod 128) / 128) in one integer
+// instruction, where exp2_neg128 extracts the exponent and applies it with
+// ldexp: 11 VALU instructions instead of 12.
+//
+// FAST: 0 <= x <= 128 * 1000 (or x negative by rounding), where every factor is
+// a normal number.  Otherwise any x >= 0: x is clamped (by its upper word)
+// where the result is 0, the reduction runs at an exponent raised by 600 and
+// one ldexp rounds into the subnormals.
+H2P_HD inline double e2x_entry(double t, int j) {
+    uint64_t b;
+    __builtin_memcpy(&b, &t, sizeof b);
+    b -= (uint64_t)j << 45;
+    __builtin_memcpy(&t, &b, sizeof t);
+    return t;
+}
+
+typedef uint32_t h2p_u2 __attribute__((vector_size(8)));   // the words of a double
+
+// c2: the second polynomial coefficient, H2P_E2X_C2; the device kernels hold it
+// in a vector register, since an FMA reads one scalar operand at most.
+#define H2P_E2X_C2 0x1.c6b09b16cfcd0p-26
+// In two halves, so that a caller can have the table reads of several values in
+// flight before the polynomials.
+struct E2X {
+    double u, T;
+    uint32_t k;
+};
+
+template <bool FAST>
+H2P_HD inline E2X exp2_neg128x_begin(double x, const double *tab) {
+    h2p_u2 b;
+    if (!FAST) {
+        __builtin_memcpy(&b, &x, sizeof b);
+        const int32_t hi = (int32_t)b[1], cl = 0x41013000;   // 128 * 1100
+        b[1] = (uint32_t)(hi < cl ? hi : cl);
+        __builtin_memcpy(&x, &b, sizeof b);
+    }
+    const double magic = 0x1.8p52 + (FAST ? 0.0 : 600.0 * 128.0);
+    const double t = magic - x;
+    const double kd = t - magic;
+    E2X e;
+    e.u = -x - kd;
+    __builtin_memcpy(&b, &t, sizeof b);
+    e.k = b[0];
+    e.T = tab[e.k & (H2P_E2_N - 1)];
+    return e;
+}
+
+template <bool FAST>
+H2P_HD inline double exp2_neg128x_end(const E2X &e, double c2) {
+    h2p_u2 b;
+    double T = e.T;
+    __builtin_memcpy(&b, &T, sizeof b);
+    b[1] += e.k << 13;
+    __builtin_memcpy(&T, &b, sizeof T);
+    double p = __builtin_fma(e.u, 0x1.3b2ab31427f87p-35, c2);
+    p = __builtin_fma(p, e.u, 0x1.ebfbdff82cc9dp-17);
+    p = __builtin_fma(p, e.u, 0x1.62e42fefa3686p-8);
+    const double r = __builtin_fma(T * e.u, p, T);
+    return FAST ? r : __builtin_ldexp(r, -600);
 }
 
 }  // namespace h2p

@@ -123,9 +123,6 @@ struct h2p_hip_handle {
     int panel_nvp = 0;
     int mm_var[4][3] = {};        // variant (task order) per matmul phase and panel width class
     int mv_var = 0;               // variant of the matvec block launch (0 default, 1 other occupancy)
-    // FP64 Gaussian / Matern JIT: the point extent can push the exponential's
-    // argument past the unclamped range, so the launches use KGW / KMW
-    bool wide = false;
     // periodic mode: shift table (x, y, z per entry; entry 0 is zero) and the
     // root's periodic block (also the matmul's dense source for the root)
     int periodic = 0;
@@ -245,23 +242,23 @@ static void launch_build(h2p_hip_handle *h, hipStream_t s) {
                            h->d_coord, h->CT, h->kp, (double *)h->d_blob);
 }
 
+// coordinate scale of the matvec's kernel-evaluating launches
+static double mv_scale(const h2p_hip_handle *h) {
+    return kscale(h->kid, h->kp.p0, h->prec == H2P_HIP_FP64);
+}
+
 // variant 0 (default): the kernel compiled for 4 waves per SIMD; variant 1:
 // compiled without an occupancy target (more registers, 2-3 waves per SIMD)
 template <int KID, typename T, int PART>
 static void launch_jit2_part(h2p_hip_handle *h, hipStream_t s, const h2p_hip_handle::BlkPart &P) {
     if (P.n == 0) return;
     const BlkTask *tasks = h->d_blk + P.off;
-    if constexpr (KID == KGW || KID == KMW) {   // one build for the clamped kernels
-        hipLaunchKernelGGL((k_blocks_jit2_occ<KID, T, 4, PART>), dim3(P.units), dim3(256), 0, s, tasks, P.big, P.n,
-                           h->d_coord, h->CT, kscale(KID, h->kp.p0, sizeof(T) == 8), h->kp.p0, h->d_xin, h->d_arena);
-        return;
-    }
     if (h->mv_var == 1)
         hipLaunchKernelGGL((k_blocks_jit2<KID, T, PART>), dim3(P.units), dim3(256), 0, s, tasks, P.big, P.n,
-                           h->d_coord, h->CT, kscale(KID, h->kp.p0, sizeof(T) == 8), h->kp.p0, h->d_xin, h->d_arena);
+                           h->d_coord, h->CT, mv_scale(h), h->kp.p0, h->d_xin, h->d_arena);
     else
         hipLaunchKernelGGL((k_blocks_jit2_occ<KID, T, 4, PART>), dim3(P.units), dim3(256), 0, s, tasks, P.big, P.n,
-                           h->d_coord, h->CT, kscale(KID, h->kp.p0, sizeof(T) == 8), h->kp.p0, h->d_xin, h->d_arena);
+                           h->d_coord, h->CT, mv_scale(h), h->kp.p0, h->d_xin, h->d_arena);
 }
 
 template <int KID, typename T>
@@ -278,12 +275,10 @@ static void dispatch_jit(h2p_hip_handle *h, hipStream_t s, int part) {
         case KC: f32 ? launch_jit2<KC, float>(h, s, part) : launch_jit2<KC, double>(h, s, part); break;
         case KG:
             if (f32) launch_jit2<KG, float>(h, s, part);
-            else if (h->wide) launch_jit2<KGW, double>(h, s, part);
             else launch_jit2<KG, double>(h, s, part);
             break;
         case KM:
             if (f32) launch_jit2<KM, float>(h, s, part);
-            else if (h->wide) launch_jit2<KMW, double>(h, s, part);
             else launch_jit2<KM, double>(h, s, part);
             break;
         default:
@@ -590,8 +585,8 @@ static void launch_mm(const h2p_hip_handle *h, int kind, const MMTask *tasks, in
     } else if (kind == MMK_JIT) {
         switch (h->kid) {
             case KC: hipLaunchKernelGGL((k_mmj<KC, NVT>), g, b, 0, s, tasks, A); break;
-            case KG: hipLaunchKernelGGL((k_mmj<KGW, NVT>), g, b, 0, s, tasks, A); break;
-            case KM: hipLaunchKernelGGL((k_mmj<KMW, NVT>), g, b, 0, s, tasks, A); break;
+            case KG: hipLaunchKernelGGL((k_mmj<KG, NVT>), g, b, 0, s, tasks, A); break;
+            case KM: hipLaunchKernelGGL((k_mmj<KM, NVT>), g, b, 0, s, tasks, A); break;
             default: hipLaunchKernelGGL((k_mmj<KR, NVT>), g, b, 0, s, tasks, A); break;
         }
     } else if (h->mode == H2P_HIP_AOT) {
@@ -810,23 +805,6 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
     }
     if (rcp_row)
         for (long long i = 0; i < CT; i++) cu[(size_t)4 * CT + i] = 1.0 / cu[(size_t)3 * CT + i];
-    // FP64 Gaussian / Matern JIT: the largest scaled distance bounds the
-    // argument of the exponential; past 2^30 the launches clamp it (wide)
-    if (mode == H2P_HIP_JIT && prec == H2P_HIP_FP64 && (krnl->id == KG || krnl->id == KM)) {
-        double ext = 0.0;
-        for (int d = 0; d < 3; d++) {
-            const double *c = cu.data() + (size_t)d * CT;
-            double lo = c[0], hi = c[0];
-            for (long long i = 1; i < CT; i++) {
-                lo = std::min(lo, c[i]);
-                hi = std::max(hi, c[i]);
-            }
-            ext = std::max(ext, hi - lo);
-        }
-        const double rmax = 1.7320508075688772 * ext * kscale(krnl->id, h->kp.p0, false);
-        const double arg = krnl->id == KG ? rmax * rmax : rmax * 1.4426950408889634;
-        h->wide = !(arg < 0x1p30);   // also for non-finite coordinates or parameters
-    }
     // ---- upward sweep tasks per level
     // level split (split handles): the tree level holding the most leaves
     // (the deepest on a tie) and everything below it are "deep"
@@ -934,11 +912,13 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
     // each node's points and of its skeleton points, from which a block knows
     // that none of its pairs is within the sum of two radii, or coincident
     // (a margin of 1e-12 covers the rounding of the kernel's own distances,
-    // and gaps below 1e-100 could still have a distance whose square is 0)
+    // and gaps below 1e-100 could still have a distance whose square is 0).
+    // FP64 Gaussian and Matern: the boxes bound a block's smallest kernel
+    // value (H2P_BLK_FAST).
     struct Extent { double lo[3], hi[3], a; };
     std::vector<Extent> ext_pt, ext_sk;
-    const bool far_flags = (krnl->id == KR || krnl->id == KC) && mode == H2P_HIP_JIT && prec == H2P_HIP_FP64;
-    if (far_flags) {
+    const bool ext_flags = mode == H2P_HIP_JIT && prec == H2P_HIP_FP64;
+    if (ext_flags) {
         auto extent = [&](long long c, int n) {
             Extent e;
             for (int d = 0; d < 3; d++) e.lo[d] = HUGE_VAL, e.hi[d] = -HUGE_VAL;
@@ -962,14 +942,21 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             if (g->U_ncol[n] > 0) ext_sk[n] = extent(g->n_point + joff[n], g->J_npt[n]);
         }
     }
-    auto far_apart = [&](const Extent &a, const Extent &b, const double *shift) {
-        double d2 = 0.0;
+    auto block_flags = [&](const Extent &a, const Extent &b, const double *shift) {
+        double gap2 = 0.0, max2 = 0.0;
         for (int d = 0; d < 3; d++) {
             const double s = shift ? shift[d] : 0.0;
             const double gap = std::max({0.0, b.lo[d] + s - a.hi[d], a.lo[d] - (b.hi[d] + s)});
-            d2 += gap * gap;
+            const double span = std::max(b.hi[d] + s - a.lo[d], a.hi[d] - (b.lo[d] + s));
+            gap2 += gap * gap;
+            max2 += span * span;
         }
-        return std::sqrt(d2) > std::max((a.a + b.a) * (1.0 + 1e-12), 1e-100);   // false for NaN
+        // every comparison is false for NaN
+        if (krnl->id == KR || krnl->id == KC)
+            return std::sqrt(gap2) > std::max((a.a + b.a) * (1.0 + 1e-12), 1e-100) ? H2P_BLK_FAR : 0;
+        const double log2e = 1.4426950408889634;
+        const double arg = krnl->id == KG ? h->kp.p0 * max2 : 1.7320508075688772 * h->kp.p0 * std::sqrt(max2);
+        return arg >= 0.0 && arg * log2e <= 1000.0 ? H2P_BLK_FAST : 0;
     };
     for (int i = 0; i < g->n_r_adm_pair; i++) {
         const int n0 = g->r_adm_pairs[2 * i], n1 = g->r_adm_pairs[2 * i + 1];
@@ -999,9 +986,9 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             t.out1 = arena; arena += t.ncol;
             (l0 > l1 ? dest_leaf[n1] : dest_y1[n1]).push_back(t.out1);
         }
-        if (far_flags && far_apart(l0 < l1 ? ext_pt[n0] : ext_sk[n0], l0 > l1 ? ext_pt[n1] : ext_sk[n1],
-                                   per ? g->per_adm_shifts + 3 * (size_t)i : nullptr))
-            t.flags |= H2P_BLK_FAR;
+        if (ext_flags)
+            t.flags |= block_flags(l0 < l1 ? ext_pt[n0] : ext_sk[n0], l0 > l1 ? ext_pt[n1] : ext_sk[n1],
+                                   per ? g->per_adm_shifts + 3 * (size_t)i : nullptr);
         B_pairs += (double)t.n0 * t.n1;
         blk.push_back(t);
         blk_deep.push_back(std::max(l0, l1) >= h->lv_cut ? 1 : 0);
@@ -1041,9 +1028,9 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             t.flags = 0;
             t.out1 = -1;
         }
-        if (far_flags && i >= nlf &&
-            far_apart(ext_pt[n0], ext_pt[n1], per ? g->per_inadm_shifts + 3 * (size_t)(i - nlf) : nullptr))
-            t.flags |= H2P_BLK_FAR;
+        if (ext_flags)
+            t.flags |= block_flags(ext_pt[n0], ext_pt[n1],
+                                   per && i >= nlf ? g->per_inadm_shifts + 3 * (size_t)(i - nlf) : nullptr);
         D_pairs += (double)t.n0 * t.n1;
         if (t.nrow == 0 || t.ncol == 0) continue;
         blk.push_back(t);
@@ -2291,7 +2278,7 @@ static MVPlan plan_matvec(TableBuf &tb, int n, h2p_hip_handle *const *hs, const 
         ReqCtx &c = reqs[i];
         c.coord = h->d_coord;
         c.CT = h->CT;
-        c.scale = kscale(h->kid, h->kp.p0, h->prec == H2P_HIP_FP64);
+        c.scale = mv_scale(h);
         c.diag = h->kp.p0;
         c.kp = h->kp;
         c.xin = h->d_xin;
@@ -2383,11 +2370,11 @@ static void launch_blocks_b(const BLaunch &b, const char *dbase, const ReqCtx *r
             break;
         case KG:
             if (f32) hipLaunchKernelGGL((k_blocks_jit2_b<KG, float, 4>), grid, blk, 0, s, it, b.n_items, reqs);
-            else hipLaunchKernelGGL((k_blocks_jit2_b<KGW, double, 4>), grid, blk, 0, s, it, b.n_items, reqs);
+            else hipLaunchKernelGGL((k_blocks_jit2_b<KG, double, 4>), grid, blk, 0, s, it, b.n_items, reqs);
             break;
         case KM:
             if (f32) hipLaunchKernelGGL((k_blocks_jit2_b<KM, float, 4>), grid, blk, 0, s, it, b.n_items, reqs);
-            else hipLaunchKernelGGL((k_blocks_jit2_b<KMW, double, 4>), grid, blk, 0, s, it, b.n_items, reqs);
+            else hipLaunchKernelGGL((k_blocks_jit2_b<KM, double, 4>), grid, blk, 0, s, it, b.n_items, reqs);
             break;
         default:
             if (f32) hipLaunchKernelGGL(k_blocks_rpy32_b, grid, blk, 0, s, it, b.n_items, reqs);
@@ -2416,8 +2403,8 @@ static void launch_mm_b(int kind, int kid, const BatchItem *it, const BLaunch &b
     } else if (kind == MMK_JIT) {
         switch (kid) {
             case KC: hipLaunchKernelGGL((k_mmj_b<KC, NVT>), g, blk, 0, s, it, n, reqs); break;
-            case KG: hipLaunchKernelGGL((k_mmj_b<KGW, NVT>), g, blk, 0, s, it, n, reqs); break;
-            case KM: hipLaunchKernelGGL((k_mmj_b<KMW, NVT>), g, blk, 0, s, it, n, reqs); break;
+            case KG: hipLaunchKernelGGL((k_mmj_b<KG, NVT>), g, blk, 0, s, it, n, reqs); break;
+            case KM: hipLaunchKernelGGL((k_mmj_b<KM, NVT>), g, blk, 0, s, it, n, reqs); break;
             default: hipLaunchKernelGGL((k_mmj_b<KR, NVT>), g, blk, 0, s, it, n, reqs); break;
         }
     } else {

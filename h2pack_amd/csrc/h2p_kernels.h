@@ -22,7 +22,7 @@ struct BlkTask {
     int c0, c1;           // JIT: first point of each set in the unified coordinates
     int n0, n1;           // JIT: point counts
     int in0, in1;         // xin offsets of the operands (in0: ncol long, in1: nrow long)
-    int flags;            // bit 0: has out1; bit 1 (H2P_BLK_FAR): the boxes of the two sets are apart
+    int flags;            // bit 0: has out1; bits 1, 2: H2P_BLK_FAR, H2P_BLK_FAST
     int shift;            // index into the shift table, added to set 1's coordinates
                           // (periodic images; entry 0 is the zero shift)
 };
@@ -30,6 +30,8 @@ struct BlkTask {
 // The two point sets' bounding boxes are apart: no coincident pair, and for
 // RPY no pair within the sum of two radii.
 #define H2P_BLK_FAR 2
+// Gaussian, Matern: no kernel value of the block is below 2^-1000.
+#define H2P_BLK_FAST 4
 
 // Upward-sweep task: y0[out] = U^T in, U row-major nrow x r.
 #define H2P_FWD_MIN_WG 256    // a level's upward tasks narrow their column chunks to reach this many (one per CU)
@@ -919,6 +921,16 @@ __global__ void __launch_bounds__(256) k_root_block(const double *__restrict__ p
 // large block; a wave unit runs four small blocks (n0 <= H2P_JITW_ROWS,
 // n1 <= 16 H2P_JITM_NT), one per wave, with wave-private LDS and no
 // workgroup barriers, so the short blocks do not wait on each other.
+// Bound by the FP64 pipe and by the wait for the table: the four values of a
+// lane's tile are evaluated together, their four table reads in flight
+// before the polynomials, and blocks whose values stay normal (H2P_BLK_FAST, 94%
+// of the pairs at N = 1M) add the exponent by an integer operation.  53 instead
+// of 57 VALU operations per tile (Matern: 85 instead of 97); matvec N = 1M
+// Gaussian 13.94 -> 13.60 ms, CG on three Matern matrices of 12-24k points
+// 6.36 -> 5.93 ms per 10 iterations.  A 1024-entry table with a polynomial of one
+// degree less (49 operations) measured slower, 14.5 ms: 8 KB of table to copy
+// per workgroup and more bank conflicts; several units per workgroup, to copy
+// it once, 14.8 ms.
 #define H2P_JITM_NT 8
 
 // Runs a tile body for the rows that hold points: lane group g's register r
@@ -937,19 +949,19 @@ struct JitmRow { double a[4]; };   // (1, x, y, z) of a target; (|s|^2, -2 s) of
 struct JitmNV { double n, v; };    // |r|^2 and the transposed product's input
 
 // LDS of the norm-form kernels, in doubles: the workgroup unit uses rows
-// (4 + 2) x H2P_JIT_ROWS, sources 5 x 16 NT and the wave partials
-// 4 x NT x 64; a wave unit gives each wave (4 + 2) x H2P_JITW_ROWS + 5 x 16 NT.
-#define H2P_JITM_LDS_WG (6 * H2P_JIT_ROWS + 5 * 16 * H2P_JITM_NT + 4 * H2P_JITM_NT * H2P_WAVE)
+// (4 + 2) x H2P_JIT_ROWS, sources 5 x 16 NT and the wave partials 4 x 16 NT; a
+// wave unit gives each wave (4 + 2) x H2P_JITW_ROWS + 5 x 16 NT.
+#define H2P_JITM_LDS_WG (6 * H2P_JIT_ROWS + 5 * 16 * H2P_JITM_NT + 4 * 16 * H2P_JITM_NT)
 #define H2P_JITM_LDS_WAVE (6 * H2P_JITW_ROWS + 5 * 16 * H2P_JITM_NT)
 #define H2P_JITM_LDS (H2P_JITM_LDS_WG > 4 * H2P_JITM_LDS_WAVE ? H2P_JITM_LDS_WG : 4 * H2P_JITM_LDS_WAVE)
 
-template <int KID, int NT, int NW>
+template <int KID, int NT, int NW, bool FAST>
 __device__ __forceinline__ void jitm_pass(const BlkTask &t, int pbase, int npts,
                                           const double *__restrict__ cx, long long cstride,
-                                          double scale, double diag, double ox, double oy, double oz,
+                                          double scale, double ox, double oy, double oz,
                                           const double *__restrict__ xin, double *__restrict__ arena,
                                           JitmRow *rowa, JitmNV *rownv, JitmRow *srcb, double *srcx,
-                                          double *red, const double *e2t, bool first) {
+                                          double *red, const double *e2x, bool first) {
     constexpr int ROWS = NW == 4 ? H2P_JIT_ROWS : H2P_JITW_ROWS;
     const int lane = threadIdx.x & 63, w = NW == 4 ? (threadIdx.x >> 6) : 0;
     const int tid = NW == 4 ? threadIdx.x : lane;
@@ -968,6 +980,8 @@ __device__ __forceinline__ void jitm_pass(const BlkTask &t, int pbase, int npts,
         srcb[q] = b;
         srcx[q] = ok ? xin[t.in0 + pbase + q] : 0.0;
     }
+    double c2 = H2P_E2X_C2;
+    asm volatile("" : "+v"(c2));   // stays in a vector register
     double acc[NT];
 #pragma unroll
     for (int c = 0; c < NT; c++) acc[c] = 0.0;
@@ -994,6 +1008,10 @@ __device__ __forceinline__ void jitm_pass(const BlkTask &t, int pbase, int npts,
         jitm_sync<NW>();
         for (int tt = w; tt < ntile; tt += NW) {
             const double a = rowa[tt * 16 + li].a[lg];
+            // one base for all tiles, opaque so that it stays one
+            unsigned o = li;
+            asm volatile("" : "+v"(o));
+            const double *sx = srcx + o, *sb = (const double *)srcb + 4 * o + lg;
             d4 cn;
             double v[4], p[4];
 #pragma unroll
@@ -1010,15 +1028,20 @@ __device__ __forceinline__ void jitm_pass(const BlkTask &t, int pbase, int npts,
                 constexpr int NR = decltype(nrq)::value;
 #pragma unroll
                 for (int c = 0; c < NT; c++) {
-                    const double xc = srcx[c * 16 + li];
-                    const d4 q = __builtin_amdgcn_mfma_f64_16x16x4f64(a, srcb[c * 16 + li].a[lg], cn, 0, 0, 0);
+                    const double xc = sx[c * 16];
+                    const d4 q = __builtin_amdgcn_mfma_f64_16x16x4f64(a, sb[c * 64], cn, 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
+                    double kv[NR];
+                    kjit<KID, FAST, NR>(q, e2x, c2, kv);
 #pragma unroll
                     for (int r = 0; r < NR; r++) {
-                        const double kv = kprep<KID>(q[r], diag, e2t);
-                        p[r] += kv * xc;
-                        acc[c] += kv * v[r];
+                        p[r] += kv[r] * xc;
+                        acc[c] += kv[r] * v[r];
                     }
+                    // Matern: pinned here, or the compiler sinks the column sums past
+                    // the row stores, keeps every kernel value alive and spills
+                    // (the Gaussian fits and is 1.5% faster left alone)
+                    if constexpr (KID == KM) asm volatile("" : "+v"(acc[c]));
                     __builtin_amdgcn_sched_barrier(0);
                 }
             };
@@ -1033,36 +1056,31 @@ __device__ __forceinline__ void jitm_pass(const BlkTask &t, int pbase, int npts,
         }
     }
     if (!has1) return;
-    if constexpr (NW == 4) {
+    // (g0 + g1) + (g2 + g3) over the four lane groups, then the waves in order
 #pragma unroll
-        for (int c = 0; c < NT; c++) red[(w * NT + c) * H2P_WAVE + lane] = acc[c];
-        __syncthreads();
-        for (int j = threadIdx.x; j < npts; j += blockDim.x) {
-            const int c = j >> 4, m = j & 15;
-            double s = 0.0;
-#pragma unroll
-            for (int w2 = 0; w2 < 4; w2++)
-#pragma unroll
-                for (int g = 0; g < 4; g++) s += red[(w2 * NT + c) * H2P_WAVE + g * 16 + m];
-            arena[t.out1 + pbase + j] = s;
-        }
-    } else {
-        // (g0 + g1) + (g2 + g3) over the four lane groups
-#pragma unroll
-        for (int c = 0; c < NT; c++) {
-            double s = acc[c] + __shfl_xor(acc[c], 16, H2P_WAVE);
-            s += __shfl_xor(s, 32, H2P_WAVE);
-            const int j = c * 16 + li;
+    for (int c = 0; c < NT; c++) {
+        double s = acc[c] + __shfl_xor(acc[c], 16, H2P_WAVE);
+        s += __shfl_xor(s, 32, H2P_WAVE);
+        const int j = c * 16 + li;
+        if constexpr (NW == 4) {
+            if (lg == 0) red[w * 16 * H2P_JITM_NT + j] = s;
+        } else {
             if (lg == 0 && j < npts) arena[t.out1 + pbase + j] = s;
         }
     }
+    if constexpr (NW == 4) {
+        constexpr int LC = 16 * H2P_JITM_NT;
+        __syncthreads();
+        for (int j = threadIdx.x; j < npts; j += blockDim.x)
+            arena[t.out1 + pbase + j] = (red[j] + red[LC + j]) + (red[2 * LC + j] + red[3 * LC + j]);
+    }
 }
 
-template <int KID, int NW>
+template <int KID, int NW, bool FAST>
 __device__ __forceinline__ void jitm_task(const BlkTask &t, const double *__restrict__ cx,
-                                          long long cstride, double scale, double diag,
+                                          long long cstride, double scale,
                                           const double *__restrict__ xin, double *__restrict__ arena,
-                                          double *lds, const double *e2t) {
+                                          double *lds, const double *e2x) {
     constexpr int ROWS = NW == 4 ? H2P_JIT_ROWS : H2P_JITW_ROWS;
     JitmRow *rowa = (JitmRow *)lds;
     JitmNV *rownv = (JitmNV *)(lds + 4 * ROWS);
@@ -1070,12 +1088,14 @@ __device__ __forceinline__ void jitm_task(const BlkTask &t, const double *__rest
     double *srcx = lds + 6 * ROWS + 4 * 16 * H2P_JITM_NT;
     double *red = srcx + 16 * H2P_JITM_NT;   // workgroup unit only
     const double ox = cx[t.c0], oy = cx[cstride + t.c0], oz = cx[2 * cstride + t.c0];
-    for (int pb = 0; pb < t.n1; pb += H2P_JITM_NT * 16) {
-        const int np = min(t.n1 - pb, H2P_JITM_NT * 16);
-        const bool first = (pb == 0);
+    const int ntile = (t.n1 + 15) >> 4, npass = (ntile + H2P_JITM_NT - 1) / H2P_JITM_NT;
+    const int per = npass > 0 ? (ntile + npass - 1) / npass : 1;   // tiles per pass, evenly
+    for (int c0 = 0; c0 < ntile; c0 += per) {
+        const int pb = 16 * c0, np = min(t.n1 - pb, 16 * per);
+        const bool first = c0 == 0;
         switch ((np + 15) >> 4) {
 #define H2P_JITM_CASE(n) \
-            case n: jitm_pass<KID, n, NW>(t, pb, np, cx, cstride, scale, diag, ox, oy, oz, xin, arena, rowa, rownv, srcb, srcx, red, e2t, first); break;
+            case n: jitm_pass<KID, n, NW, FAST>(t, pb, np, cx, cstride, scale, ox, oy, oz, xin, arena, rowa, rownv, srcb, srcx, red, e2x, first); break;
             H2P_JITM_CASE(1) H2P_JITM_CASE(2) H2P_JITM_CASE(3) H2P_JITM_CASE(4)
             H2P_JITM_CASE(5) H2P_JITM_CASE(6) H2P_JITM_CASE(7) H2P_JITM_CASE(8)
 #undef H2P_JITM_CASE
@@ -1087,23 +1107,28 @@ __device__ __forceinline__ void jitm_task(const BlkTask &t, const double *__rest
 
 // Launch unit u of a tiled launch: u < nbig runs task u on the whole
 // workgroup, later units run tasks nbig + 4 (u - nbig) + w, one per wave.
-// The exp2_neg table is copied into LDS first (one copy per workgroup).
+// The exp2_neg128x table is copied into LDS first (one copy per workgroup).
 template <int KID>
 __device__ __forceinline__ void blocks_jitm_unit(const BlkTask *__restrict__ tasks, int u, int nbig, int ntask,
                                                  const double *__restrict__ cx, long long cstride,
-                                                 double scale, double diag, const double *__restrict__ xin,
+                                                 double scale, const double *__restrict__ xin,
                                                  double *__restrict__ arena) {
     __shared__ double lds[H2P_JITM_LDS];
-    __shared__ double e2t[H2P_E2_N];
-    if (threadIdx.x < H2P_E2_N) e2t[threadIdx.x] = c_e2tab[threadIdx.x];
+    __shared__ double e2x[H2P_E2_N];
+    if (threadIdx.x < H2P_E2_N) e2x[threadIdx.x] = e2x_entry(c_e2tab[threadIdx.x], threadIdx.x);
     __syncthreads();
     if (u < nbig) {
-        jitm_task<KID, 4>(tasks[u], cx, cstride, scale, diag, xin, arena, lds, e2t);
+        const BlkTask t = tasks[u];
+        if (t.flags & H2P_BLK_FAST) jitm_task<KID, 4, true>(t, cx, cstride, scale, xin, arena, lds, e2x);
+        else jitm_task<KID, 4, false>(t, cx, cstride, scale, xin, arena, lds, e2x);
     } else {
-        const int w = threadIdx.x >> 6;
+        const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         const int i = nbig + 4 * (u - nbig) + w;
-        if (i < ntask)
-            jitm_task<KID, 1>(tasks[i], cx, cstride, scale, diag, xin, arena, lds + w * H2P_JITM_LDS_WAVE, e2t);
+        if (i >= ntask) return;
+        const BlkTask t = tasks[i];
+        double *l = lds + w * H2P_JITM_LDS_WAVE;
+        if (t.flags & H2P_BLK_FAST) jitm_task<KID, 1, true>(t, cx, cstride, scale, xin, arena, l, e2x);
+        else jitm_task<KID, 1, false>(t, cx, cstride, scale, xin, arena, l, e2x);
     }
 }
 
@@ -1456,8 +1481,8 @@ __device__ __forceinline__ void blocks_jit2_unit(const BlkTask *__restrict__ tas
                                                  double *__restrict__ arena) {
     if constexpr (sizeof(T) == 4) {
         blocks_jitf_unit<KID>(tasks, u, nbig, ntask, cx, cstride, scale, diag, xin, arena);
-    } else if constexpr (KID == KG || KID == KM || KID == KGW || KID == KMW) {
-        blocks_jitm_unit<KID>(tasks, u, nbig, ntask, cx, cstride, scale, diag, xin, arena);
+    } else if constexpr (KID == KG || KID == KM) {
+        blocks_jitm_unit<KID>(tasks, u, nbig, ntask, cx, cstride, scale, xin, arena);
     } else {
         static_assert(KID == KC, "scalar kernels only");
         blocks_jitc_unit(tasks, u, nbig, ntask, cx, cstride, diag, xin, arena);

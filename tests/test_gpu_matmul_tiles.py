@@ -49,3 +49,18 @@ def test_wide_point_set_matches_oracle(kid):
     Y = H2MatHIP(h2, mode="jit").matmul(X, "col")
     # coordinates of 1e6 leave differences 1e-10 absolute: the bar is theirs
     assert np.isfinite(Y).all() and rel(Y, ref) < 1e-9
+
+
+@pytest.mark.parametrize("kid", [C.KRNL_GAUSSIAN, C.KRNL_MATERN32])
+@pytest.mark.parametrize("scale", [1.0, 12.0, 60.0])
+def test_matvec_underflowing_blocks_match_oracle(kid, scale):
+    """Blocks whose kernel values stay normal take the short exponential, those
+    that can underflow the other: trees with none, some and many of the latter."""
+    rng = np.random.default_rng(8)
+    coord = rng.random((3, 3000)) * 6.0 * scale
+    h2 = C.build_h2(coord, kid, [1.0], 1e-8, 90, BD_JIT=1, pp_kind="surface", host_blocks=False)
+    x = rng.random(h2.krnl_mat_size) - 0.5
+    ref = O.OracleH2(h2, BD_JIT=1).matvec(x, n_thread=8)
+    m = H2MatHIP(h2, mode="jit")
+    assert rel(m.matvec(x), ref) < 1e-12
+    m.close()
