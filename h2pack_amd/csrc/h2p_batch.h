@@ -131,7 +131,7 @@ __global__ void __launch_bounds__(256) k_leaf_final2_b(const BatchItem *__restri
     const int it = find_item(items, n, blockIdx.x);
     const ReqCtx &c = reqs[items[it].req];
     const LeafTask2 t = ((const LeafTask2 *)items[it].tasks)[blockIdx.x - items[it].begin];
-    leaf_final2_body(t, c.contrib, c.arena, c.UT, c.yp, c.fwd, c.y, c.xin, c.shift);
+    leaf_final2_body(t, c.contrib, c.arena, c.UT, c.y1, c.yp, c.fwd, c.y, c.xin, c.shift);
 }
 
 // ---------------------------------------------------------------------------

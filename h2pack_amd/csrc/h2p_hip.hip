@@ -409,7 +409,7 @@ static void launch_interior(h2p_hip_handle *h, hipStream_t s, hipEvent_t *ev) {
     if (ev) (void)hipEventRecord(ev[5], s);
     if (h->split)
         hipLaunchKernelGGL(k_leaf_u, dim3(h->n_leaf), dim3(256), 0, s, h->d_leaf, h->d_contrib, h->d_arena, h->d_UT,
-                           h->d_yp, h->d_yt);
+                           h->d_y1, h->d_yp, h->d_yt);
     if (fork) (void)hipStreamWaitEvent(s, h->ev_join, 0);
 }
 
@@ -420,7 +420,7 @@ static void launch_leaf_out(h2p_hip_handle *h, double *d_y, hipStream_t s) {
                            h->d_yt, h->d_fwd, d_y, (const double *)h->d_xin, 0.0);
     else
         hipLaunchKernelGGL(k_leaf_final2, dim3(h->n_leaf), dim3(256), 0, s, h->d_leaf, h->d_contrib, h->d_arena,
-                           h->d_UT, h->d_yp, h->d_fwd, d_y, (const double *)h->d_xin, 0.0);
+                           h->d_UT, h->d_y1, h->d_yp, h->d_fwd, d_y, (const double *)h->d_xin, 0.0);
 }
 
 // Point the graph's gather node at x and its leaf-output node at y.  The
@@ -446,15 +446,15 @@ static int graph_set_xy(h2p_hip_handle *h, const double *d_x, double *d_y) {
         const long long *a1 = h->d_contrib;
         const double *a2 = h->d_arena;
         const double *a3 = h->split ? (const double *)h->d_yt : (const double *)h->d_UT;
-        const double *a4 = h->d_yp;
+        const double *a4 = h->d_y1, *a4p = h->d_yp;
         const int *a5 = h->d_fwd;
         double *a6 = d_y;
         const double *a7 = h->d_xin;
         double a8 = 0.0;
         void *split_args[] = {(void *)&a0, (void *)&a1, (void *)&a2, (void *)&a3, (void *)&a5, (void *)&a6,
                               (void *)&a7, (void *)&a8};
-        void *final_args[] = {(void *)&a0, (void *)&a1, (void *)&a2, (void *)&a3, (void *)&a4, (void *)&a5,
-                              (void *)&a6, (void *)&a7, (void *)&a8};
+        void *final_args[] = {(void *)&a0, (void *)&a1, (void *)&a2, (void *)&a3, (void *)&a4, (void *)&a4p,
+                              (void *)&a5, (void *)&a6, (void *)&a7, (void *)&a8};
         p.kernelParams = h->split ? split_args : final_args;
         p.extra = nullptr;
         HIP_TRY(hipGraphExecKernelNodeSetParams(h->graph_exec, h->gnode_leaf, &p));
@@ -826,12 +826,12 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
         // workgroup keeps the same loads in flight at any width, so more of
         // them on a small level means more bytes in flight)
         int ncol = 4 * H2P_WAVE;
-        while (ncol > H2P_WAVE) {
+        while (ncol > 16) {
             long long nwg = 0;
             for (int j = 0; j < g->level_n_node[lv]; j++)
                 nwg += (g->U_ncol[g->level_nodes[(size_t)lv * nlf + j]] + ncol - 1) / ncol;
             if (nwg >= H2P_FWD_MIN_WG) break;
-            ncol >>= 1;
+            ncol = ncol == H2P_WAVE ? 16 : ncol >> 1;
         }
         for (int j = 0; j < g->level_n_node[lv]; j++) {
             int n = g->level_nodes[(size_t)lv * nlf + j];
@@ -1100,34 +1100,65 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             active[n] = ((g->node_n_r_adm[n] > 0 || has_push[n] || per_root) && g->U_ncol[n] > 0) ? 1 : 0;
             if (!active[n]) has_push[n] = 0;
         }
-    // ---- non-leaf skeleton sums (leaves sum their own in the output kernel)
+    // chunk width of a launch over outputs of the given lengths: the widest
+    // with at least min_wg workgroups (see group_sum)
+    auto chunk_width = [](const std::vector<int> &len, const std::array<int, 2> &min_wg) {
+        for (int k = 0; k < 2; k++) {
+            const int w = k == 0 ? 256 : 64;
+            long long nwg = 0;
+            for (int v : len) nwg += (v + w - 1) / w;
+            if (nwg >= min_wg[k]) return w;
+        }
+        return 16;
+    };
+    // ---- skeleton sums.  The leaves' are summed with the inner nodes' but
+    // in two cases, where the output kernel sums them: a tree without inner
+    // nodes to sum (saves the launch), and split handles (the sums would wait
+    // for the D blocks' workgroups in a launch of their own).
     // (the nodes above lv_cut first: on a split handle their sums belong to
     // the shallow levels' chain)
     std::vector<long long> contrib;
     std::vector<RedTask> red;
-    for (int pass = 0; pass < 2; pass++)
+    bool leaf_own = true;
+    for (int n = 0; n < nn; n++)
+        if (g->U_ncol[n] > 0 && g->n_child[n] > 0) leaf_own = h->split;
+    for (int pass = 0; pass < 2; pass++) {
+        std::vector<int> nodes, len;
         for (int n = 0; n < nn; n++) {
-            if (g->U_ncol[n] == 0 || g->n_child[n] == 0) continue;
+            if (g->U_ncol[n] == 0 || (g->n_child[n] == 0 && (leaf_own || !active[n]))) continue;
             if ((g->node_level[n] < h->lv_cut) != (pass == 0)) continue;
+            nodes.push_back(n);
+            len.push_back(g->U_ncol[n]);
+        }
+        const int w = chunk_width(len, H2P_RED_MIN_WG);
+        for (int n : nodes) {
             RedTask t{};
             t.dst = soff[n];
             t.len = g->U_ncol[n];
+            t.w = w;
             t.cbeg = (int)contrib.size();
             for (long long o : dest_y1[n]) contrib.push_back(o);
             t.cend = (int)contrib.size();
-            red.push_back(t);
-            if (pass == 0) h->n_red_shallow++;
+            for (t.e0 = 0; t.e0 < t.len; t.e0 += w) red.push_back(t);
         }
+        if (pass == 0) h->n_red_shallow = (int)red.size();
+    }
     h->n_red = (int)red.size();
-    // ---- downward sweep: one task per 256-row chunk, level by level
+    // ---- downward sweep: one task per row chunk, level by level
     std::vector<BwdTask2> bwdt;
     for (int lv = g->min_adm_level; lv <= g->max_level; lv++) {
         Level L{(int)bwdt.size(), 0};
+        std::vector<int> len;
+        for (int j = 0; j < g->level_n_node[lv]; j++) {
+            int n = g->level_nodes[(size_t)lv * nlf + j];
+            if (active[n] && g->n_child[n] > 0) len.push_back(g->U_nrow[n]);
+        }
+        const int w = chunk_width(len, H2P_BWD_MIN_WG);
         for (int j = 0; j < g->level_n_node[lv]; j++) {
             int n = g->level_nodes[(size_t)lv * nlf + j];
             if (!active[n] || g->n_child[n] == 0) continue;
             if (g->U_ncol[n] > H2P_MAXR) return bail(fail(H2P_HIP_ENOSYS, "rank above 2048"));
-            for (int r0 = 0; r0 < g->U_nrow[n]; r0 += 256) {
+            for (int r0 = 0; r0 < g->U_nrow[n]; r0 += w) {
                 BwdTask2 t{};
                 t.ut_off = uoff[n];
                 t.nrow = g->U_nrow[n];
@@ -1136,6 +1167,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
                 t.push = has_push[n];
                 t.out_off = soff[g->children[(size_t)n * mc]];
                 t.row0 = r0;
+                t.w = w;
                 bwdt.push_back(t);
             }
         }
@@ -1146,6 +1178,11 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
         }
     }
     std::vector<LeafTask2> leaf;
+    std::vector<int> leaf_len;
+    for (int i = 0; i < nlf; i++) leaf_len.push_back(npt(g->leaf_nodes[i]) * kd);
+    int leaf_w = leaf_own ? chunk_width(leaf_len, H2P_LEAF_OWN_MIN_WG) : chunk_width(leaf_len, H2P_LEAF_MIN_WG);
+    // many small leaves: 64 rows are one chunk of a leaf all the same
+    if (leaf_own && leaf_w == 256 && *std::max_element(leaf_len.begin(), leaf_len.end()) <= 64) leaf_w = 64;
     for (int i = 0; i < nlf; i++) {
         int n = g->leaf_nodes[i];
         LeafTask2 t{};
@@ -1156,14 +1193,16 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
         t.ut_off = uoff[n];
         t.s_off = soff[n];
         t.vec_s = g->mat_cluster[2 * n];
+        t.own = leaf_own;
+        t.w = leaf_w;
         t.cb1 = (int)contrib.size();
-        if (t.r > 0)
+        if (t.r > 0 && leaf_own)
             for (long long o : dest_y1[n]) contrib.push_back(o);
         t.ce1 = (int)contrib.size();
         t.cb0 = (int)contrib.size();
         for (long long o : dest_leaf[n]) contrib.push_back(o);
         t.ce0 = (int)contrib.size();
-        leaf.push_back(t);
+        for (t.row0 = 0; t.row0 < t.nrow; t.row0 += leaf_w) leaf.push_back(t);
     }
     h->n_leaf = (int)leaf.size();
     // ---- matmul tasks (pull form, one task per destination)
@@ -1376,23 +1415,25 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
         const long long BLOB = (long long)(btot + dtot);
         if (XIN > 0x7fffffffLL) return bail(fail(H2P_HIP_EINVAL, "vector space exceeds 2^31 entries"));
         auto in = [](long long off, long long len, long long cap) { return off >= 0 && len >= 0 && off + len <= cap; };
+        auto width_ok = [](int w) { return w == 256 || w == 64 || w == 16; };
         for (const FwdTask &t : fwdt)
             if (!in(t.in_off, t.nrow, XIN) || !in(t.out_off, t.r, XIN) || !in(t.u_off, (long long)t.nrow * t.r, utot) ||
-                t.col0 < 0 || t.col0 >= t.r || (t.ncol != 64 && t.ncol != 128 && t.ncol != 256))
+                t.col0 < 0 || t.col0 >= t.r || (t.ncol != 16 && t.ncol != 64 && t.ncol != 128 && t.ncol != 256))
                 return bail(fail(H2P_HIP_EINVAL, "upward task out of range"));
         for (const BwdTask2 &t : bwdt)
             if (!in(t.y1_off, t.r, Y1) || !in(t.out_off, t.nrow, Y1) || !in(t.ut_off, (long long)t.nrow * t.r, utot) ||
-                t.row0 < 0 || t.row0 >= t.nrow || t.r > H2P_MAXR)
+                t.row0 < 0 || t.row0 >= t.nrow || t.r > H2P_MAXR || !width_ok(t.w))
                 return bail(fail(H2P_HIP_EINVAL, "downward task out of range"));
         for (const RedTask &t : red) {
-            if (!in(t.dst, t.len, Y1) || t.cbeg < 0 || t.cend < t.cbeg || t.cend > NC)
+            if (!in(t.dst, t.len, Y1) || t.cbeg < 0 || t.cend < t.cbeg || t.cend > NC || t.e0 < 0 ||
+                t.e0 >= t.len || !width_ok(t.w))
                 return bail(fail(H2P_HIP_EINVAL, "reduction task out of range"));
             for (int k = t.cbeg; k < t.cend; k++)
                 if (!in(contrib[k], t.len, AR)) return bail(fail(H2P_HIP_EINVAL, "reduction source out of range"));
         }
         for (const LeafTask2 &t : leaf) {
             if (!in(t.vec_s, t.nrow, N) || t.cb1 < 0 || t.ce1 < t.cb1 || t.cb0 != t.ce1 || t.ce0 < t.cb0 ||
-                t.ce0 > NC || t.r > H2P_MAXR)
+                t.ce0 > NC || t.r > H2P_MAXR || t.row0 < 0 || t.row0 >= t.nrow || !width_ok(t.w))
                 return bail(fail(H2P_HIP_EINVAL, "leaf task out of range"));
             if (t.r > 0 && (!in(t.s_off, t.r, Y1) || !in(t.ut_off, (long long)t.nrow * t.r, utot)))
                 return bail(fail(H2P_HIP_EINVAL, "leaf task out of range"));

@@ -34,17 +34,25 @@ struct BlkTask {
 #define H2P_BLK_FAST 4
 
 // Upward-sweep task: y0[out] = U^T in, U row-major nrow x r.
-#define H2P_FWD_MIN_WG 256    // a level's upward tasks narrow their column chunks to reach this many (one per CU)
+// Workgroups that a launch has to reach with a chunk width, else it takes the
+// next narrower one (see group_sum): {256, 64} outputs, then 16.
+#define H2P_FWD_MIN_WG 256    // upward sweep (256, 128 and 64 columns, then 16)
+#define H2P_RED_MIN_WG {1024, 256}
+#define H2P_BWD_MIN_WG {512, 256}
+#define H2P_LEAF_MIN_WG {1024, 256}
+#define H2P_LEAF_OWN_MIN_WG {256, 256}   // every chunk sums the leaf's partials again
 struct FwdTask {
     long long u_off;
     int nrow, r, in_off, out_off;
     int col0;         // first of the output columns this task computes
-    int ncol;         // at most this many columns from col0: 64, 128 or 256
+    int ncol;         // at most this many columns from col0: 16, 64, 128 or 256
 };
 
-// Segmented reduction into y1: y1[dst + e] = sum_k arena[contrib[k] + e].
+// Segmented reduction into y1: y1[dst + e] = sum_k arena[contrib[k] + e] for
+// the w elements from e0 (e < len).
 struct RedTask {
     int dst, len, cbeg, cend;
+    int e0, w;        // w: 256, 64 or 16
 };
 
 // ---------------------------------------------------------------------------
@@ -54,11 +62,11 @@ __global__ void k_gather(const double *__restrict__ x, const int *__restrict__ i
     if (i < n) out[i] = x[idx[i]];
 }
 
-// Fixed-order segmented reduction of the block partials into y1.
 // v + arena[contrib[k] + e] for k = kb, kb + step, ... < ke, added in list
 // order.  The offsets and values of H2P_GATHER_AHEAD entries are loaded
 // before their adds, so that many loads are in flight instead of one
-// offset-then-value chain per entry; the sum is the plain loop's, bit for bit.
+// offset-then-value chain per entry; the last batch repeats the last entry
+// and adds zeros for it.
 #define H2P_GATHER_AHEAD 8
 __device__ __forceinline__ double ordered_gather_sum(double v, const long long *__restrict__ contrib,
                                                      const double *__restrict__ arena, int kb, int ke, int step,
@@ -71,14 +79,120 @@ __device__ __forceinline__ double ordered_gather_sum(double v, const long long *
 #pragma unroll
         for (int u = 0; u < H2P_GATHER_AHEAD; u++) v += a[u];
     }
-    for (; k < ke; k += step) v += arena[contrib[k] + e];
+    if (k < ke) {
+        double a[H2P_GATHER_AHEAD];
+#pragma unroll
+        for (int u = 0; u < H2P_GATHER_AHEAD; u++) {
+            const int ku = k + u * step;
+            const double x = arena[contrib[ku < ke ? ku : k] + e];
+            a[u] = ku < ke ? x : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < H2P_GATHER_AHEAD; u++) v += a[u];
+    }
     return v;
+}
+
+// The sweeps and sums below give every workgroup of 256 threads a chunk of W
+// consecutive outputs and deal the terms of each output's sum to 256 / W
+// groups of threads, whose sums are added in group order.  W = 256 (one
+// thread per output) is the least overhead where a launch has enough
+// workgroups; a level of a few nodes with long sums takes W = 64 or 16 so
+// that all CUs have loads in flight and the chain of dependent batches is
+// short (the host picks W per launch; 16 doubles are one 128-byte line).
+// The sweeps are bound by HBM where a level has hundreds of nodes and by
+// the chain of one workgroup's loads where it has a few.  us per matvec, 256
+// rows a workgroup everywhere -> widths by launch: periodic RPY N = 10k 807
+// -> 591, RPY N = 20k 472 -> 431, 10 CG iterations on three Matern matrices
+// of 24k points and fewer 5927 -> 5640.  Widths 256 / 64 / 16 of the downward
+// sweep of RPY N = 20k (64 nodes x 938 rows): 462 / 442 / 460; of the leaf
+// outputs of the periodic matrix (64 leaves x 469 rows) 64 / 16: 597 / 605.
+//
+// The group sums of one output, added in group order; valid in threads < W.
+template <int W>
+__device__ __forceinline__ double group_sum(double v, double *part) {
+    if constexpr (W == 256) return v;
+    __syncthreads();   // part may still be read by an earlier call
+    part[threadIdx.x] = v;
+    __syncthreads();
+    double s = part[threadIdx.x & (W - 1)];
+#pragma unroll
+    for (int g = 1; g < 256 / W; g++) s += part[g * W + (threadIdx.x & (W - 1))];
+    return s;
+}
+
+// group of a thread; wave-uniform (and said so) from W = 64 on
+template <int W>
+__device__ __forceinline__ int group_of() {
+    return W >= H2P_WAVE ? __builtin_amdgcn_readfirstlane(threadIdx.x / W) : threadIdx.x / W;
+}
+
+// sum_i M[i * ld] v[i] over i < n for this thread's column (M points at it):
+// each group takes a contiguous range of i, 16 values loaded before their
+// FMAs; the last batch repeats the last entry with factors of zero.  ok:
+// the thread has a column (a wave without one skips the loads).
+template <int W>
+__device__ __forceinline__ double group_dot(const double *__restrict__ M, int ld, int n, const double *v, bool ok,
+                                            double *part) {
+    constexpr int G = 256 / W;
+    const int q = (n + G - 1) / G, i0 = group_of<W>() * q, i1 = min(n, i0 + q);
+    double a0 = 0.0, a1 = 0.0;
+    if (ok) {
+        int i = i0;
+        for (; i + 15 < i1; i += 16) {
+            double u[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) u[j] = M[(long long)(i + j) * ld];
+#pragma unroll
+            for (int j = 0; j < 16; j += 2) {
+                a0 += u[j] * v[i + j];
+                a1 += u[j + 1] * v[i + j + 1];
+            }
+        }
+        for (; i < i1; i += 8) {
+            double u[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) u[j] = M[(long long)min(i + j, i1 - 1) * ld];
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                const bool k0 = i + j < i1, k1 = i + j + 1 < i1;
+                a0 += (k0 ? u[j] : 0.0) * (k0 ? v[i + j] : 0.0);
+                a1 += (k1 ? u[j + 1] : 0.0) * (k1 ? v[i + j + 1] : 0.0);
+            }
+        }
+    }
+    return group_sum<W>(a0 + a1, part);
+}
+
+// The contributions [kb, ke) of element e, dealt to the groups in turn.
+template <int W>
+__device__ __forceinline__ double group_gather(const long long *__restrict__ contrib, const double *__restrict__ arena,
+                                               int kb, int ke, int e, bool ok, double *part) {
+    double v = 0.0;
+    if (ok) v = ordered_gather_sum(0.0, contrib, arena, kb + group_of<W>(), ke, 256 / W, e);
+    return group_sum<W>(v, part);
+}
+
+#define H2P_BY_WIDTH(w, F, ...)        \
+    do {                               \
+        if ((w) == 256) F<256>(__VA_ARGS__); \
+        else if ((w) == 64) F<64>(__VA_ARGS__); \
+        else F<16>(__VA_ARGS__);       \
+    } while (0)
+
+// Fixed-order segmented reduction of the block partials into y1.
+template <int W>
+__device__ __forceinline__ void reduce_y1_w(const RedTask &t, const long long *__restrict__ contrib,
+                                            const double *__restrict__ arena, double *__restrict__ y1, double *part) {
+    const int e = t.e0 + (threadIdx.x & (W - 1));
+    const double v = group_gather<W>(contrib, arena, t.cbeg, t.cend, e, e < t.len, part);
+    if (threadIdx.x < W && e < t.len) y1[t.dst + e] = v;
 }
 
 __device__ __forceinline__ void reduce_y1_body(const RedTask &t, const long long *__restrict__ contrib,
                                                const double *__restrict__ arena, double *__restrict__ y1) {
-    for (int e = threadIdx.x; e < t.len; e += blockDim.x)
-        y1[t.dst + e] = ordered_gather_sum(0.0, contrib, arena, t.cbeg, t.cend, 1, e);
+    __shared__ double part[256];
+    H2P_BY_WIDTH(t.w, reduce_y1_w, t, contrib, arena, y1, part);
 }
 
 __global__ void __launch_bounds__(256) k_reduce_y1(const RedTask *__restrict__ tasks,
@@ -164,6 +278,12 @@ __device__ __forceinline__ void fwd2_strips(const FwdTask &t, const double *__re
 __device__ __forceinline__ void fwd2_body(const FwdTask &t, const double *__restrict__ U,
                                           double *__restrict__ xin) {
     __shared__ double red[4][4][H2P_WAVE];
+    if (t.ncol == 16) {   // 16 columns x 16 groups of rows
+        const int c = t.col0 + (threadIdx.x & 15);
+        const double v = group_dot<16>(U + t.u_off + c, t.r, t.nrow, xin + t.in_off, c < t.r, &red[0][0][0]);
+        if (threadIdx.x < 16 && c < t.r) xin[t.out_off + c] = v;
+        return;
+    }
     const int ns = (min(t.r - t.col0, t.ncol) + H2P_WAVE - 1) / H2P_WAVE;
     if (ns <= 1) fwd2_strips<1>(t, U, xin, red);
     else if (ns == 2) fwd2_strips<2>(t, U, xin, red);
@@ -177,55 +297,35 @@ __global__ void __launch_bounds__(256) k_fwd2(const FwdTask *__restrict__ tasks,
     fwd2_body(tasks[blockIdx.x], U, xin);
 }
 
-// Downward sweep (src/H2Pack_matvec.c:767-861), one workgroup per 256-row chunk of a node:
-// yp[child rows] = U (y1 + yp)[node], U^T stored row-major.  The push-down
-// buffer yp is written exactly once per row (each child has one parent).
+// Downward sweep (src/H2Pack_matvec.c:767-861), one workgroup per w-row chunk of a node:
+// yp[child rows] = U (y1 + yp)[node], U^T stored row-major, so that the lanes'
+// rows are contiguous for each column.  The push-down buffer yp is written
+// exactly once per row (each child has one parent).
 struct BwdTask2 {
     long long ut_off;
     int nrow, r, y1_off, push, out_off, row0;
+    int w, pad;       // w: 256, 64 or 16
 };
 #define H2P_MAXR 2048
-// sum_c UT[c * ld] * yv[c] for one row of U (U^T stored row-major, so the
-// lanes' rows are contiguous for each c): four accumulators taking every
-// fourth c, 16 values loaded before their FMAs; each accumulator's FMAs run
-// over its c in order, so the sum is the same for any unrolling.
-__device__ __forceinline__ double ut_row_dot(const double *__restrict__ ut, int ld, int r, const double *yv) {
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-    int c = 0;
-    for (; c + 15 < r; c += 16) {
-        double u[16];
-#pragma unroll
-        for (int j = 0; j < 16; j++) u[j] = ut[(long long)(c + j) * ld];
-#pragma unroll
-        for (int j = 0; j < 16; j += 4) {
-            a0 += u[j] * yv[c + j];
-            a1 += u[j + 1] * yv[c + j + 1];
-            a2 += u[j + 2] * yv[c + j + 2];
-            a3 += u[j + 3] * yv[c + j + 3];
-        }
-    }
-    for (; c + 3 < r; c += 4) {
-        a0 += ut[(long long)c * ld] * yv[c];
-        a1 += ut[(long long)(c + 1) * ld] * yv[c + 1];
-        a2 += ut[(long long)(c + 2) * ld] * yv[c + 2];
-        a3 += ut[(long long)(c + 3) * ld] * yv[c + 3];
-    }
-    for (; c < r; c++) a0 += ut[(long long)c * ld] * yv[c];
-    return (a0 + a1) + (a2 + a3);
+
+template <int W>
+__device__ __forceinline__ void bwd2_w(const BwdTask2 &t, const double *__restrict__ UT, const double *yv,
+                                       double *__restrict__ yp, double *part) {
+    const int row = t.row0 + (threadIdx.x & (W - 1));
+    const double v = group_dot<W>(UT + t.ut_off + row, t.nrow, t.r, yv, row < t.nrow, part);
+    if (threadIdx.x < W && row < t.nrow) yp[t.out_off + row] = v;
 }
 
 __device__ __forceinline__ void bwd2_body(const BwdTask2 &t, const double *__restrict__ UT,
                                           const double *__restrict__ y1, double *__restrict__ yp) {
-    __shared__ double yv[H2P_MAXR];
+    __shared__ double yv[H2P_MAXR], part[256];
     for (int c = threadIdx.x; c < t.r; c += blockDim.x)
         yv[c] = y1[t.y1_off + c] + (t.push ? yp[t.y1_off + c] : 0.0);
     __syncthreads();
-    const int row = t.row0 + threadIdx.x;
-    if (row >= t.nrow) return;
-    yp[t.out_off + row] = ut_row_dot(UT + t.ut_off + row, t.nrow, t.r, yv);
+    H2P_BY_WIDTH(t.w, bwd2_w, t, UT, yv, yp, part);
 }
 
-__global__ void __launch_bounds__(256) k_bwd2(const BwdTask2 *__restrict__ tasks,
+__global__ void __launch_bounds__(256, 8) k_bwd2(const BwdTask2 *__restrict__ tasks,
                                               const double *__restrict__ UT,
                                               const double *__restrict__ y1,
                                               double *__restrict__ yp) {
@@ -233,29 +333,37 @@ __global__ void __launch_bounds__(256) k_bwd2(const BwdTask2 *__restrict__ tasks
 }
 
 // Leaf outputs (src/H2Pack_matvec.c:767-861 for the leaves, and the backward
-// permutation y[fwd[i]] = py[i] of src/H2Pack_matvec.c:1156-1159): the leaf's skeleton value is its own block
-// partials plus its parent's push-down; then U y1 plus the point partials
-// go straight to the caller's order.
+// permutation y[fwd[i]] = py[i] of src/H2Pack_matvec.c:1156-1159), one
+// workgroup per w-row chunk of a leaf: the leaf's skeleton value is its
+// block partials plus its parent's push-down; then U y1 plus the point
+// partials go straight to the caller's order.  The skeleton partials were
+// summed into y1 with the inner nodes' (own = 0), or, in a tree whose leaves
+// are all there is to sum, are summed here (own = 1), which saves a launch.
 struct LeafTask2 {
     long long ut_off;
     int nrow, r, s_off, push, vec_s;
-    int cb1, ce1;   // contributions in skeleton space (length r)
+    int cb1, ce1;   // contributions in skeleton space (length r; own = 1)
     int cb0, ce0;   // contributions in point space (length nrow)
-    int pad;
+    int own, row0;
+    int w;          // 256, 64 or 16
 };
+// A leaf's output row i is
+//   (U y1)_i + (its point-space contributions) + shift x_i;
 // shift != 0 adds shift * x (a diagonal nugget applied outside the H2
 // product, as the PCG wrapper of examples/SPDHSS-H2/pcg_tests.c:15-21 does);
-// px holds x in the permuted order.  A leaf's output row i is
-//   ((U y1)_i) + its point-space contributions, in list order, + shift x_i,
-// where y1 = push-down value + skeleton-space contributions, in list order.
-// With a small rank (r <= blockDim / 2) the contributions are dealt to
-// G = blockDim / r groups of r threads (group g sums contributions g, g + G,
-// ...), so that G loads are in flight per skeleton entry instead of one
-// dependent chain, and the G group sums are added in group order; part
-// holds blockDim doubles.  The caller synchronises before reading yv.
+// px holds x in the permuted order.
+// own = 1 with a small rank (r <= blockDim / 2): the contributions are dealt
+// to G = blockDim / r groups of r threads (group g sums contributions g,
+// g + G, ...), and the G group sums are added in group order; part holds
+// blockDim doubles.  The caller synchronises before reading yv.
 __device__ __forceinline__ void leaf_stage_y1(const LeafTask2 &t, const long long *__restrict__ contrib,
-                                              const double *__restrict__ arena, const double *__restrict__ yp,
-                                              double *yv, double *part) {
+                                              const double *__restrict__ arena, const double *__restrict__ y1,
+                                              const double *__restrict__ yp, double *yv, double *part) {
+    if (!t.own) {
+        for (int c = threadIdx.x; c < t.r; c += blockDim.x)
+            yv[c] = y1[t.s_off + c] + (t.push ? yp[t.s_off + c] : 0.0);
+        return;
+    }
     const int G = t.r > 0 ? min(8, (int)blockDim.x / t.r) : 1;
     if (G <= 1) {
         for (int c = threadIdx.x; c < t.r; c += blockDim.x)
@@ -272,41 +380,60 @@ __device__ __forceinline__ void leaf_stage_y1(const LeafTask2 &t, const long lon
     }
 }
 
+template <int W>
 __device__ __forceinline__ double leaf_u_row(const LeafTask2 &t, const double *__restrict__ UT, const double *yv,
-                                             int i) {
-    return ut_row_dot(UT + t.ut_off + i, t.nrow, t.r, yv);
+                                             double *part) {
+    const int row = t.row0 + (threadIdx.x & (W - 1));
+    return group_dot<W>(UT + t.ut_off + row, t.nrow, t.r, yv, row < t.nrow, part);
 }
 
-__device__ __forceinline__ double leaf_d_row(const LeafTask2 &t, const long long *__restrict__ contrib,
+// the output row of thread < W from its U part u
+template <int W>
+__device__ __forceinline__ void leaf_out_row(const LeafTask2 &t, const long long *__restrict__ contrib,
                                              const double *__restrict__ arena, const double *__restrict__ px,
-                                             double shift, int i, double v) {
-    v = ordered_gather_sum(v, contrib, arena, t.cb0, t.ce0, 1, i);
-    if (shift != 0.0) v += shift * px[t.vec_s + i];
-    return v;
+                                             double shift, const int *__restrict__ fwd, double *__restrict__ y,
+                                             double u, double *part) {
+    const int row = t.row0 + (threadIdx.x & (W - 1));
+    const double d = group_gather<W>(contrib, arena, t.cb0, t.ce0, row, row < t.nrow, part);
+    if (threadIdx.x < W && row < t.nrow) {
+        double v = u + d;
+        if (shift != 0.0) v += shift * px[t.vec_s + row];
+        y[fwd[t.vec_s + row]] = v;
+    }
+}
+
+template <int W>
+__device__ __forceinline__ void leaf_final2_w(const LeafTask2 &t, const long long *__restrict__ contrib,
+                                              const double *__restrict__ arena, const double *__restrict__ UT,
+                                              const double *yv, const int *__restrict__ fwd, double *__restrict__ y,
+                                              const double *__restrict__ px, double shift, double *part) {
+    const double u = leaf_u_row<W>(t, UT, yv, part);
+    leaf_out_row<W>(t, contrib, arena, px, shift, fwd, y, u, part);
 }
 
 __device__ __forceinline__ void leaf_final2_body(const LeafTask2 &t, const long long *__restrict__ contrib,
                                                  const double *__restrict__ arena,
                                                  const double *__restrict__ UT,
+                                                 const double *__restrict__ y1,
                                                  const double *__restrict__ yp,
                                                  const int *__restrict__ fwd, double *__restrict__ y,
                                                  const double *__restrict__ px, double shift) {
     __shared__ double yv[H2P_MAXR], part[256];
-    leaf_stage_y1(t, contrib, arena, yp, yv, part);
+    leaf_stage_y1(t, contrib, arena, y1, yp, yv, part);
     __syncthreads();
-    for (int i = threadIdx.x; i < t.nrow; i += blockDim.x)
-        y[fwd[t.vec_s + i]] = leaf_d_row(t, contrib, arena, px, shift, i, leaf_u_row(t, UT, yv, i));
+    H2P_BY_WIDTH(t.w, leaf_final2_w, t, contrib, arena, UT, yv, fwd, y, px, shift, part);
 }
 
-__global__ void __launch_bounds__(256) k_leaf_final2(const LeafTask2 *__restrict__ tasks,
+__global__ void __launch_bounds__(256, 8) k_leaf_final2(const LeafTask2 *__restrict__ tasks,
                                                      const long long *__restrict__ contrib,
                                                      const double *__restrict__ arena,
                                                      const double *__restrict__ UT,
+                                                     const double *__restrict__ y1,
                                                      const double *__restrict__ yp,
                                                      const int *__restrict__ fwd,
                                                      double *__restrict__ y,
                                                      const double *__restrict__ px, double shift) {
-    leaf_final2_body(tasks[blockIdx.x], contrib, arena, UT, yp, fwd, y, px, shift);
+    leaf_final2_body(tasks[blockIdx.x], contrib, arena, UT, y1, yp, fwd, y, px, shift);
 }
 
 // The leaf outputs in two launches, for handles whose D blocks are still
@@ -314,16 +441,34 @@ __global__ void __launch_bounds__(256) k_leaf_final2(const LeafTask2 *__restrict
 // the permuted order, no D contribution needed), k_leaf_d adds the
 // point-space contributions once the D blocks are done.  Same operations in
 // the same order as k_leaf_final2, so the same bits.
-__global__ void __launch_bounds__(256) k_leaf_u(const LeafTask2 *__restrict__ tasks,
+template <int W>
+__device__ __forceinline__ void leaf_u_w(const LeafTask2 &t, const double *__restrict__ UT, const double *yv,
+                                         double *__restrict__ yt, double *part) {
+    const double u = leaf_u_row<W>(t, UT, yv, part);
+    const int row = t.row0 + (threadIdx.x & (W - 1));
+    if (threadIdx.x < W && row < t.nrow) yt[t.vec_s + row] = u;
+}
+
+__global__ void __launch_bounds__(256, 8) k_leaf_u(const LeafTask2 *__restrict__ tasks,
                                                 const long long *__restrict__ contrib,
                                                 const double *__restrict__ arena,
                                                 const double *__restrict__ UT,
+                                                const double *__restrict__ y1,
                                                 const double *__restrict__ yp, double *__restrict__ yt) {
     __shared__ double yv[H2P_MAXR], part[256];
     const LeafTask2 t = tasks[blockIdx.x];
-    leaf_stage_y1(t, contrib, arena, yp, yv, part);
+    leaf_stage_y1(t, contrib, arena, y1, yp, yv, part);
     __syncthreads();
-    for (int i = threadIdx.x; i < t.nrow; i += blockDim.x) yt[t.vec_s + i] = leaf_u_row(t, UT, yv, i);
+    H2P_BY_WIDTH(t.w, leaf_u_w, t, UT, yv, yt, part);
+}
+
+template <int W>
+__device__ __forceinline__ void leaf_d_w(const LeafTask2 &t, const long long *__restrict__ contrib,
+                                         const double *__restrict__ arena, const double *__restrict__ px,
+                                         double shift, const int *__restrict__ fwd, double *__restrict__ y,
+                                         const double *__restrict__ yt, double *part) {
+    const int row = min(t.row0 + (int)(threadIdx.x & (W - 1)), t.nrow - 1);
+    leaf_out_row<W>(t, contrib, arena, px, shift, fwd, y, yt[t.vec_s + row], part);
 }
 
 __global__ void __launch_bounds__(256) k_leaf_d(const LeafTask2 *__restrict__ tasks,
@@ -332,9 +477,9 @@ __global__ void __launch_bounds__(256) k_leaf_d(const LeafTask2 *__restrict__ ta
                                                 const double *__restrict__ yt,
                                                 const int *__restrict__ fwd, double *__restrict__ y,
                                                 const double *__restrict__ px, double shift) {
+    __shared__ double part[256];
     const LeafTask2 t = tasks[blockIdx.x];
-    for (int i = threadIdx.x; i < t.nrow; i += blockDim.x)
-        y[fwd[t.vec_s + i]] = leaf_d_row(t, contrib, arena, px, shift, i, yt[t.vec_s + i]);
+    H2P_BY_WIDTH(t.w, leaf_d_w, t, contrib, arena, px, shift, fwd, y, yt, part);
 }
 
 // ---------------------------------------------------------------------------
