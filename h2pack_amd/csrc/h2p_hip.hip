@@ -78,6 +78,15 @@ inline bool fwdidx_ok(int v, int n) { return v >= 0 && v < n; }
 
 // profiling events recorded per matvec call (see launch_interior)
 #define H2P_EV_PER_CALL 7
+// A JIT handle with fewer kernel pairs than this runs its matvec in order on
+// one stream, all blocks in one launch: each wait for another stream costs
+// 5 to 9 us and each launch of a few blocks about 10 us, which the overlap
+// with the sweeps only wins back on larger trees.  us per matvec, streams /
+// in order: Gaussian N = 4k (8e6 pairs) 57.6 / 38.7, 16k (1.2e8) 151.8 /
+// 135.0, 24k (2.0e8) 223.8 / 214.0, 40k (3.6e8) 359 / 372, 64k (6.6e8) 593 /
+// 632; Coulomb 24k (1.0e8) 152 / 142, 64k (3.8e8) 360 / 378; Matern
+// FP32-mixed 24k (1.7e8) 170 / 156, 64k (7.2e8) 471 / 497.
+#define H2P_ONE_LAUNCH_PAIRS 2.5e8
 // share of the D blocks' kernel pairs launched after the B blocks (the
 // smallest blocks), overlapping the skeleton sums and the downward sweep;
 // the rest overlaps the upward sweep.  H2P_HIP_D_LATE overrides it.
@@ -139,6 +148,9 @@ struct h2p_hip_handle {
     // workgroup-unit tasks first
     struct BlkPart { int off = 0, n = 0, big = 0, units = 0; };
     BlkPart part[4];
+    // small split handles: all parts once more as one launch (a copy of the
+    // tasks behind the parts), used while everything runs in order
+    BlkPart all;
     bool split = false;             // D blocks on aux_stream, concurrent with the sweeps
     bool d_serial = false;          // split handle whose D blocks run in order (h2p_hip_autotune)
     hipStream_t aux_stream = nullptr;
@@ -261,11 +273,13 @@ static void launch_jit2_part(h2p_hip_handle *h, hipStream_t s, const h2p_hip_han
                            h->d_coord, h->CT, mv_scale(h), h->kp.p0, h->d_xin, h->d_arena);
 }
 
+#define H2P_PART_ALL 4
 template <int KID, typename T>
 static void launch_jit2(h2p_hip_handle *h, hipStream_t s, int part) {
     // the B parts (0, 3) share one kernel instantiation (template argument
-    // 0), the D parts (1, 2) another
-    if (part == 0 || part == 3) launch_jit2_part<KID, T, 0>(h, s, h->part[part]);
+    // 0) with the launch of all blocks, the D parts (1, 2) another
+    if (part == H2P_PART_ALL) launch_jit2_part<KID, T, 0>(h, s, h->all);
+    else if (part == 0 || part == 3) launch_jit2_part<KID, T, 0>(h, s, h->part[part]);
     else launch_jit2_part<KID, T, 1>(h, s, h->part[part]);
 }
 
@@ -362,7 +376,23 @@ static void launch_reduce(h2p_hip_handle *h, hipStream_t s, int t0, int t1) {
                            h->d_y1);
 }
 
+// True when a handle's matvec runs in order with all blocks in one launch;
+// the leaf outputs are then one launch too.  Calls with profiling events run
+// the parts one by one, with the same results.
+static bool one_launch(const h2p_hip_handle *h, const hipEvent_t *ev) {
+    return h->all.n > 0 && h->d_serial && !h->lv_on && !ev;
+}
+
+static bool leaf_in_two(const h2p_hip_handle *h, const hipEvent_t *ev) { return h->split && !one_launch(h, ev); }
+
 static void launch_interior(h2p_hip_handle *h, hipStream_t s, hipEvent_t *ev) {
+    if (one_launch(h, ev)) {
+        launch_fwd(h, s, 0, (int)h->fwd_levels.size());
+        dispatch_jit(h, s, H2P_PART_ALL);
+        launch_reduce(h, s, 0, h->n_red);
+        launch_bwd(h, s, 0, (int)h->bwd_levels.size());
+        return;
+    }
     const bool fork = h->split && !h->d_serial && !ev && (h->part[1].n > 0 || h->part[2].n > 0);
     const bool lv = h->split && h->lv_on && h->lv_possible && !ev;
     const int nf = (int)h->fwd_levels.size(), nbw = (int)h->bwd_levels.size();
@@ -414,8 +444,8 @@ static void launch_interior(h2p_hip_handle *h, hipStream_t s, hipEvent_t *ev) {
 }
 
 // The leaf outputs of a matvec into the caller's y (the last launch).
-static void launch_leaf_out(h2p_hip_handle *h, double *d_y, hipStream_t s) {
-    if (h->split)
+static void launch_leaf_out(h2p_hip_handle *h, double *d_y, hipStream_t s, const hipEvent_t *ev) {
+    if (leaf_in_two(h, ev))
         hipLaunchKernelGGL(k_leaf_d, dim3(h->n_leaf), dim3(256), 0, s, h->d_leaf, h->d_contrib, h->d_arena,
                            h->d_yt, h->d_fwd, d_y, (const double *)h->d_xin, 0.0);
     else
@@ -445,7 +475,8 @@ static int graph_set_xy(h2p_hip_handle *h, const double *d_x, double *d_y) {
         const LeafTask2 *a0 = h->d_leaf;
         const long long *a1 = h->d_contrib;
         const double *a2 = h->d_arena;
-        const double *a3 = h->split ? (const double *)h->d_yt : (const double *)h->d_UT;
+        const bool two = leaf_in_two(h, nullptr);
+        const double *a3 = two ? (const double *)h->d_yt : (const double *)h->d_UT;
         const double *a4 = h->d_y1, *a4p = h->d_yp;
         const int *a5 = h->d_fwd;
         double *a6 = d_y;
@@ -455,7 +486,7 @@ static int graph_set_xy(h2p_hip_handle *h, const double *d_x, double *d_y) {
                               (void *)&a7, (void *)&a8};
         void *final_args[] = {(void *)&a0, (void *)&a1, (void *)&a2, (void *)&a3, (void *)&a4, (void *)&a4p,
                               (void *)&a5, (void *)&a6, (void *)&a7, (void *)&a8};
-        p.kernelParams = h->split ? split_args : final_args;
+        p.kernelParams = two ? split_args : final_args;
         p.extra = nullptr;
         HIP_TRY(hipGraphExecKernelNodeSetParams(h->graph_exec, h->gnode_leaf, &p));
         h->graph_y = d_y;
@@ -471,7 +502,7 @@ static int ensure_graph(h2p_hip_handle *h, const double *d_x, double *d_y) {
     HIP_TRY(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
     hipLaunchKernelGGL(k_gather, dim3((h->N + 255) / 256), dim3(256), 0, cs, d_x, h->d_fwd, h->d_xin, h->N);
     launch_interior(h, cs, nullptr);
-    launch_leaf_out(h, d_y, cs);
+    launch_leaf_out(h, d_y, cs, nullptr);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(cs, &g);
     if (e != hipSuccess) return fail(H2P_HIP_EDEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
@@ -480,7 +511,7 @@ static int ensure_graph(h2p_hip_handle *h, const double *d_x, double *d_y) {
     std::vector<hipGraphNode_t> nodes(n);
     HIP_TRY(hipGraphGetNodes(g, nodes.data(), &n));
     const void *f_gather = reinterpret_cast<const void *>(&k_gather);
-    const void *f_leaf = h->split ? reinterpret_cast<const void *>(&k_leaf_d)
+    const void *f_leaf = leaf_in_two(h, nullptr) ? reinterpret_cast<const void *>(&k_leaf_d)
                                   : reinterpret_cast<const void *>(&k_leaf_final2);
     hipGraphNode_t ng = nullptr, nl = nullptr;
     int n_gather = 0, n_leaf = 0;
@@ -544,7 +575,7 @@ static int run_matvec(h2p_hip_handle *h, const double *d_x, double *d_y, hipStre
     if (prof) HIP_TRY(hipEventRecord(ev[0], s));
     hipLaunchKernelGGL(k_gather, dim3((h->N + 255) / 256), dim3(256), 0, s, d_x, h->d_fwd, h->d_xin, h->N);
     launch_interior(h, s, ev);
-    launch_leaf_out(h, d_y, s);
+    launch_leaf_out(h, d_y, s, ev);
     HIP_TRY(hipGetLastError());
     if (prof) {
         HIP_TRY(hipEventRecord(ev[6], s));
@@ -1054,8 +1085,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
     h->part[3].n = h->split ? nB - nB_deep : 0;
     h->part[1].off = h->split ? nB : h->n_blk;
     h->part[1].n = h->n_blk - h->part[1].off;
-    for (int k : {0, 3, 1}) {
-        auto &P = h->part[k];
+    auto order_part = [&](h2p_hip_handle::BlkPart &P) {
         auto b0 = blk.begin() + P.off, b1 = b0 + P.n;
         std::stable_sort(b0, b1, [](const BlkTask &x, const BlkTask &y) {
             return (long long)x.nrow * x.ncol > (long long)y.nrow * y.ncol;
@@ -1065,7 +1095,8 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             P.big = (int)(std::stable_partition(b0, b1, [&](const BlkTask &t) { return !wave_task(t); }) -
                           b0);
         P.units = P.big + (P.n - P.big + 3) / 4;
-    }
+    };
+    for (int k : {0, 3, 1}) order_part(h->part[k]);
     // the D blocks' last tasks (the smallest, about d_late of their pairs)
     // form part 2, launched after the B blocks
     if (h->split && h->part[1].n > 0) {
@@ -1087,6 +1118,15 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
         P2.n = D.n - cut;
         P2.big = std::max(0, D.big - cut);
         P2.units = P2.big + (P2.n - P2.big + 3) / 4;
+    }
+    // a small handle's blocks once more, in one list (H2P_ONE_LAUNCH_PAIRS)
+    h->all = h2p_hip_handle::BlkPart{};
+    if (h->split && h->n_blk > 0 && B_pairs + D_pairs < H2P_ONE_LAUNCH_PAIRS) {
+        auto &P = h->all;
+        P.off = P.n = h->n_blk;
+        blk.insert(blk.end(), blk.begin(), blk.begin() + h->n_blk);
+        order_part(P);
+        h->d_serial = true;
     }
     // ---- active nodes of the downward sweep (y1 "set", src/H2Pack_matvec.c:251-256, :802-838)
     std::vector<char> active(nn, 0), has_push(nn, 0);
@@ -1588,7 +1628,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
     }
     h->h_mmt = std::move(mmt);
     h->h_mms = std::move(mms);
-    h->h_blk = blk;
+    h->h_blk.assign(blk.begin(), blk.begin() + h->n_blk);
     // FP32-mixed handles without FP32 matmul tiles (RPY, whose matmul tiles
     // are FP64 only) refuse matmul rather than run it in FP64
     h->mm_ok = !(prec == H2P_HIP_FP32MIX && !mm_f32);
@@ -1656,7 +1696,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
              hipEventCreateWithFlags(&h->ev_lv, hipEventDisableTiming) != hipSuccess ||
              hipEventCreateWithFlags(&h->ev_side, hipEventDisableTiming) != hipSuccess))
             return bail(fail(H2P_HIP_EDEVICE, "level-split stream / event create failed"));
-        h->lv_on = h->lv_possible;
+        h->lv_on = h->all.n > 0 ? 0 : h->lv_possible;
     }
     // the upload is synchronous: callers may use the handle on any stream,
     // including streams that do not order with the null stream
@@ -1948,14 +1988,20 @@ int h2p_hip_matmul(h2p_hip_handle *h, int layout, int n_vec, const double *X, in
 // have taken host faults).
 static int time_interior(h2p_hip_handle *h, int reps, double *ms) {
     hipStream_t s = h->own_stream;
-    launch_interior(h, s, nullptr);   // warm-up
+    // the leaves' U y1 rows are part of the interior of a split schedule and
+    // of the leaf outputs (here into yt, which these do not read) of the other
+    auto interior = [&] {
+        launch_interior(h, s, nullptr);
+        if (one_launch(h, nullptr)) launch_leaf_out(h, h->d_yt, s, nullptr);
+    };
+    interior();   // warm-up
     HIP_TRY(hipGetLastError());
     hipEvent_t e0 = nullptr, e1 = nullptr;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     float t = 0.f;
     int rc = hipEventRecord(e0, s) == hipSuccess ? 0 : fail(H2P_HIP_EDEVICE, "hipEventRecord failed");
-    for (int r = 0; r < reps && !rc; r++) launch_interior(h, s, nullptr);
+    for (int r = 0; r < reps && !rc; r++) interior();
     if (!rc && (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                 hipEventElapsedTime(&t, e0, e1) != hipSuccess))
         rc = fail(H2P_HIP_EDEVICE, "timing the matvec interior failed");
