@@ -29,6 +29,20 @@ struct KParam {
     double p1;      // RPY: C = 1/(6 pi eta); others unused
 };
 
+// Correctly rounded sqrt(q) of a squared distance in FP32 (q >= 0, below
+// 1e-30 as 1e-30; infinity gives NaN): the hardware reciprocal root and one
+// correction s += y/2 (q - s^2), which gives the rounded root for every
+// mantissa and both parities of the exponent (compared over [1, 4)).  The
+// library's takes 15 operations around the hardware root, for denormals and
+// signs that a squared distance does not have.
+__device__ __forceinline__ float sqrt_q(float q) {
+    const unsigned b = __builtin_bit_cast(unsigned, q), fl = 0x0da24260u;   // 1e-30
+    const float qq = __builtin_bit_cast(float, b > fl ? b : fl);
+    const float y = __builtin_amdgcn_rsqf(qq);
+    const float s = qq * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, qq), 0.5f * y, s);
+}
+
 // Scalar kernels as functions of r^2 (kd = 1).
 template <int KID>
 __device__ __forceinline__ double kval(double r2, const KParam &kp) {
@@ -50,7 +64,7 @@ __device__ __forceinline__ float kvalf(float r2, float p0) {
         // exp(-l r2) = 2^(-l r2 log2 e)
         return __builtin_amdgcn_exp2f(-p0 * 1.4426950408889634f * r2);
     } else {
-        float t = -1.7320508075688772f * p0 * __builtin_sqrtf(r2);
+        float t = -1.7320508075688772f * p0 * sqrt_q(r2);
         return (1.0f - t) * __builtin_amdgcn_exp2f(t * 1.4426950408889634f);
     }
 }
