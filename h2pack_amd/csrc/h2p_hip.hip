@@ -1151,6 +1151,11 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
         }
         return 16;
     };
+    // larger split handles run these launches beside block launches that fill
+    // the chip, where more and smaller workgroups only delay the blocks
+    // (Matern FP32-mixed N = 105k: 729 us with narrower chunks, 713 with 256;
+    // Coulomb N = 200k the other way round, 1397 and 1412)
+    const bool beside = h->split && h->all.n == 0;
     // ---- skeleton sums.  The leaves' are summed with the inner nodes' but
     // in two cases, where the output kernel sums them: a tree without inner
     // nodes to sum (saves the launch), and split handles (the sums would wait
@@ -1170,7 +1175,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             nodes.push_back(n);
             len.push_back(g->U_ncol[n]);
         }
-        const int w = chunk_width(len, H2P_RED_MIN_WG);
+        const int w = beside ? 256 : chunk_width(len, H2P_RED_MIN_WG);
         for (int n : nodes) {
             RedTask t{};
             t.dst = soff[n];
@@ -1193,7 +1198,7 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
             int n = g->level_nodes[(size_t)lv * nlf + j];
             if (active[n] && g->n_child[n] > 0) len.push_back(g->U_nrow[n]);
         }
-        const int w = chunk_width(len, H2P_BWD_MIN_WG);
+        const int w = beside ? 256 : chunk_width(len, H2P_BWD_MIN_WG);
         for (int j = 0; j < g->level_n_node[lv]; j++) {
             int n = g->level_nodes[(size_t)lv * nlf + j];
             if (!active[n] || g->n_child[n] == 0) continue;
