@@ -191,32 +191,44 @@ __device__ __forceinline__ double sqrt_floored(double q) {
     return __builtin_fma(g * e, __builtin_fma(0.375, e, 0.5), g);
 }
 
-// Scalar kernels on prepared squared distances.  Coordinates are scaled
-// before the distance is formed so that the kernels need no parameter:
-//   Gaussian exp(-l r^2)          : scale sqrt(128 l log2 e) -> K = 2^(-q / 128)
-//   Matern32 (1+t) e^{-t}, t=sqrt3 l r : scale sqrt3 l       -> K = (1+s) e^(-s), s = sqrt(q)
-//   Coulomb 1/r                   : scale 1                  -> K = q == 0 ? diag : rsqrt(q)
-// (kscale(kid, p0, true)).  e2t is the exp2_neg128 table (LDS), unused by
-// Coulomb.
+// Scalar kernels of the FP64 matmul on r^2 from coordinate differences, c the
+// kernel's factor (kmm_scale):
+//   Gaussian exp(-l r^2)               : c = 128 l log2 e -> K = 2^(-c r^2 / 128)
+//   Matern32 (1+t) e^{-t}, t=sqrt3 l r : c = sqrt3 l, s = c r -> K = (1+s) e^(-s)
+//   Coulomb 1/r                        : K = r^2 == 0 ? diag : rsqrt(r^2)
+// The factor is applied to r^2 (Matern: to r), not to the coordinates, whose
+// rounding would count against their differences.  e2t is the exp2_neg128
+// table (LDS), unused by Coulomb.
+__host__ __device__ inline double kmm_scale(int kid, double p0) {
+    if (kid == KG) return 128.0 * 1.4426950408889634 * p0;
+    if (kid == KM) return 1.7320508075688772 * p0;
+    return 1.0;
+}
+
 template <int KID>
-__device__ __forceinline__ double kprep(double q, double diag, const double *e2t = nullptr) {
+__device__ __forceinline__ double kmm(double r2, double c, double diag, const double *e2t) {
     if constexpr (KID == KC) {
-        const bool z = q == 0.0;
-        const double y = rsqrt_refined(z ? 1.0 : q);   // branch-free
+        const bool z = r2 == 0.0;
+        const double y = rsqrt_refined(z ? 1.0 : r2);   // branch-free
         return z ? diag : y;
     } else if constexpr (KID == KG) {
-        return exp2_neg128_clamped(q, e2t);
+        return exp2_neg128_clamped(r2 * c, e2t);
     } else {
         static_assert(KID == KM, "scalar kernels only");
-        const double s = sqrt_floored(q);
+        const double s = sqrt_floored(r2) * c;
         const double x = s * (128.0 * 1.4426950408889634);   // e^(-s) = 2^(-x / 128)
         const double e = exp2_neg128_clamped(x, e2t);
         return __builtin_fma(s, e, e);
     }
 }
 
-// The same for the matvec's norm-form launches, NR values at once (so that NR
-// table reads are in flight); FAST as for exp2_neg128x.
+// Scalar kernels of the matvec's launches on prepared squared distances:
+// coordinates are scaled before the distance is formed so that the kernels
+// need no parameter (kscale):
+//   Gaussian exp(-l r^2)               : scale sqrt(128 l log2 e) -> K = 2^(-q / 128)
+//   Matern32 (1+t) e^{-t}, t=sqrt3 l r : scale sqrt3 l            -> K = (1+s) e^(-s), s = sqrt(q)
+// FP64 (norm form), NR values at once (so that NR table reads are in
+// flight); FAST as for exp2_neg128x.
 template <int KID, bool FAST, int NR>
 __device__ __forceinline__ void kjit(const d4 &q, const double *e2x, double c2, double *kv) {
     static_assert(KID == KG || KID == KM, "norm-form kernels only");

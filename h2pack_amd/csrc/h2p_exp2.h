@@ -3,7 +3,7 @@
 // function in IEEE floating-point arithmetic", ACM TOMS 15(2), 1989, here in
 // base 2 with 128 table entries).  Used by the FP64 Gaussian and Matern-3/2
 // kernel evaluations of the matmul, whose arguments arrive
-// already multiplied by 128 (the Gaussian through its coordinate scale);
+// already multiplied by 128 (through the kernel's factor);
 // the reference evaluates the same kernels through its SIMD library's exp
 // (src/H2Pack_3D_kernels.h:212-268, 433-497).
 //

@@ -598,7 +598,7 @@ static MMArgs mm_args(const h2p_hip_handle *h, const MMPanels &P) {
     A.cx = h->d_coord;
     A.cstride = h->CT;
     A.shifts = h->d_shift;
-    A.scale = kscale(h->kid, h->kp.p0, true);
+    A.scale = kmm_scale(h->kid, h->kp.p0);
     A.kp = h->kp;
     A.P = P;
     return A;

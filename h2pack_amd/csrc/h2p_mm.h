@@ -31,12 +31,10 @@
 //   dense A    : step r, lane group g take entry 4 g + r, so a lane reads 32
 //                consecutive bytes of its row (transposed blocks: each step
 //                reads 16 consecutive rows' entries, 128 bytes per group);
-//   evaluated A: step r, lane group g take entry 4 r + g.  The tile of
-//                squared distances q[src][dst] of 16 sources x 16
-//                destinations is itself one MFMA whose result register r holds
-//                source 4 r + g against destination l % 16, exactly the A
-//                operand of step r: kernel values go from the evaluation into
-//                the product without leaving the lane.
+//   evaluated A: step r, lane group g take entry 4 r + g.  A lane evaluates
+//                source 4 r + g against destination l % 16 for r = 0 .. 3,
+//                the A operands of the four steps: kernel values go from the
+//                evaluation into the product without leaving the lane.
 #pragma once
 #include "h2p_device.h"
 
@@ -85,7 +83,7 @@ struct MMArgs {
     const double *cx;          // unified coordinates, one row per dimension
     long long cstride;
     const double *shifts;
-    double scale;              // coordinate scale of the FP64 norm-form kernels
+    double scale;              // the FP64 kernels' factor (kmm_scale)
     KParam kp;
     MMPanels P;
 };
@@ -228,41 +226,38 @@ __device__ __forceinline__ void mm_dense(const MMTask &t, int sbeg, int send, co
 }
 
 // The evaluated sources of a task, scalar kernels: 16 sources x 32
-// destinations per chunk, distances by MFMA (Gaussian, Matern; coordinates
-// relative to the task's first destination point, pre-scaled as in the
-// matvec) or from coordinate differences (Coulomb, whose r = 0 must be
-// exact), kernel values straight into the products.
+// destinations per chunk, kernel values straight into the products.  The
+// distances are coordinate differences on the VALU (6 operations a pair): a
+// leaf or a skeleton can hold points far apart, and |r|^2 + |s|^2 - 2 r.s,
+// one matrix product for the tile, is off by the square of its extent
+// (times 2^-53): two groups of a leaf 8e4 lengthscales apart gave products off
+// by 1e-7, now 1e-15, and 7.6e-15 -> 5.0e-16 for Matern points in a cube of
+// side 10 (l = 2).  us per product, squares -> differences: Gaussian
+// N = 40k x16 1153 -> 1296, N = 17k x64 959 -> 1035; Matern 1383 -> 1556 and
+// 960 -> 1029.
 template <int KID, int NVT, bool GUARD>
 __device__ __forceinline__ void mm_jit1(const MMTask &t, const MMArgs &A, int nt, int w, int li, int lg,
                                         const double *e2t, d4 (*acc)[NVT]) {
-    constexpr bool NORM = KID != KC;
     const double *cx = A.cx, *cy = A.cx + A.cstride, *cz = A.cx + 2 * A.cstride;
     const double scale = A.scale, diag = A.kp.p0;
-    const double ox = NORM ? cx[t.c0] : 0.0, oy = NORM ? cy[t.c0] : 0.0, oz = NORM ? cz[t.c0] : 0.0;
     MMCursor<16> cu;
     cu.start(A.srcs, t.smid, t.send, w);
     if (!cu.live()) return;
-    // destinations of the two tiles: point 16 q + li (the B operand (1, r)
-    // and the accumulator input |r|^2, or the plain coordinates)
-    double db[2], dx[2], dy[2], dz[2];
-    d4 dn[2];
+    // destinations of the two tiles: point 16 q + li
+    double dx[2], dy[2], dz[2];
 #pragma unroll
     for (int q = 0; q < 2; q++) {
         const int g = t.c0 + min(16 * q + li, t.M - 1);
-        dx[q] = (cx[g] - ox) * scale;
-        dy[q] = (cy[g] - oy) * scale;
-        dz[q] = (cz[g] - oz) * scale;
-        const double nn = mm_sq3(dx[q], dy[q], dz[q]);
-        dn[q] = (d4){nn, nn, nn, nn};
-        db[q] = lg == 0 ? 1.0 : lg == 1 ? dx[q] : lg == 2 ? dy[q] : dz[q];
+        dx[q] = cx[g];
+        dy[q] = cy[g];
+        dz[q] = cz[g];
     }
-    // sources of a chunk: point li (norm form) or points 4 r + lg
-    constexpr int NC = NORM ? 1 : 4;
-    double sx[NC], sy[NC], sz[NC];
+    // sources of a chunk: points 4 r + lg
+    double sx[4], sy[4], sz[4];
     auto fetch = [&](const MMSrc &s, int c) {
 #pragma unroll
-        for (int r = 0; r < NC; r++) {
-            const int g = s.c1 + min(16 * c + (NORM ? li : 4 * r + lg), s.K - 1);
+        for (int r = 0; r < 4; r++) {
+            const int g = s.c1 + min(16 * c + 4 * r + lg, s.K - 1);
             sx[r] = cx[g];
             sy[r] = cy[g];
             sz[r] = cz[g];
@@ -274,33 +269,21 @@ __device__ __forceinline__ void mm_jit1(const MMTask &t, const MMArgs &A, int nt
         double x[4][NVT];
         mm_load_x<NVT, GUARD>(A.P.p[cu.s.x_space] + (long long)cu.s.x_off * A.P.nvp, A.P.nvp, nt, cu.s.K, 16 * cu.c,
                               lg, 4, li, x);
-        double px[NC], py[NC], pz[NC];
+        double px[4], py[4], pz[4];
 #pragma unroll
-        for (int r = 0; r < NC; r++) {
+        for (int r = 0; r < 4; r++) {
             px[r] = sx[r];
             py[r] = sy[r];
             pz[r] = sz[r];
         }
         cu.next(A.srcs);
         if (cu.live()) fetch(cu.s, cu.c);
-        double sa = 0.0;
-        if constexpr (NORM) {
-            const double ux = (px[0] - ox) * scale, uy = (py[0] - oy) * scale, uz = (pz[0] - oz) * scale;
-            const double nn = mm_sq3(ux, uy, uz);
-            sa = lg == 0 ? nn : -2.0 * (lg == 1 ? ux : lg == 2 ? uy : uz);
-        }
         auto tile = [&](int q) {
-            d4 d2;
-            if constexpr (NORM) d2 = __builtin_amdgcn_mfma_f64_16x16x4f64(sa, db[q], dn[q], 0, 0, 0);
             double kv[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                if constexpr (NORM) {
-                    kv[r] = kprep<KID>(d2[r], diag, e2t);
-                } else {
-                    const double ex = dx[q] - px[r], ey = dy[q] - py[r], ez = dz[q] - pz[r];
-                    kv[r] = kprep<KID>(mm_sq3(ex, ey, ez), diag);
-                }
+                const double ex = dx[q] - px[r], ey = dy[q] - py[r], ez = dz[q] - pz[r];
+                kv[r] = kmm<KID>(mm_sq3(ex, ey, ez), scale, diag, e2t);
             }
 #pragma unroll
             for (int r = 0; r < 4; r++)
