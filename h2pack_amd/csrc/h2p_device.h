@@ -29,19 +29,10 @@ struct KParam {
     double p1;      // RPY: C = 1/(6 pi eta); others unused
 };
 
-// Correctly rounded sqrt(q) of a squared distance in FP32 (q >= 0, below
-// 1e-30 as 1e-30; infinity gives NaN): the hardware reciprocal root and one
-// correction s += y/2 (q - s^2), which gives the rounded root for every
-// mantissa and both parities of the exponent (compared over [1, 4)).  The
-// library's takes 15 operations around the hardware root, for denormals and
-// signs that a squared distance does not have.
-__device__ __forceinline__ float sqrt_q(float q) {
-    const unsigned b = __builtin_bit_cast(unsigned, q), fl = 0x0da24260u;   // 1e-30
-    const float qq = __builtin_bit_cast(float, b > fl ? b : fl);
-    const float y = __builtin_amdgcn_rsqf(qq);
-    const float s = qq * y;
-    return __builtin_fmaf(__builtin_fmaf(-s, s, qq), 0.5f * y, s);
-}
+// sqrt(q) of a squared distance in FP32 from the hardware reciprocal root
+// (sqrt_from_rsq).  The library's takes 15 operations around the hardware
+// root, for denormals and signs that a squared distance does not have.
+__device__ __forceinline__ float sqrt_q(float q) { return sqrt_from_rsq(q, __builtin_amdgcn_rsqf(q)); }
 
 // Scalar kernels as functions of r^2 (kd = 1).
 template <int KID>

@@ -167,4 +167,20 @@ H2P_HD inline double exp2_neg128x_end(const E2X &e, double c2) {
     return FAST ? r : __builtin_ldexp(r, -600);
 }
 
+// sqrt(q) of a squared distance in FP32 from an estimate y of 1/sqrt(q): s = q y
+// and one correction s += y/2 (q - s^2).  An estimate that is right to a unit in
+// the last place gives the root to (1/2 + 2^-18) units; below q = 2^-102, where
+// the correction's residual is subnormal, to 3/4 unit.  y is clipped to 2^63, its
+// value at the smallest normal q, so that q = 0 gives 0 and a subnormal q,
+// where the hardware's estimate is infinity, a root of at most 2^-63.
+// Infinity gives NaN.
+H2P_HD inline float sqrt_from_rsq(float q, float y) {
+    int32_t b;
+    __builtin_memcpy(&b, &y, sizeof b);
+    b = b < 0x5f000000 ? b : 0x5f000000;   // 2^63
+    __builtin_memcpy(&y, &b, sizeof y);
+    const float s = q * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, q), 0.5f * y, s);
+}
+
 }  // namespace h2p
