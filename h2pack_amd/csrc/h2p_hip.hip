@@ -1985,31 +1985,31 @@ int h2p_hip_matmul(h2p_hip_handle *h, int layout, int n_vec, const double *X, in
     return rc;
 }
 
-// Mean time of the matvec interior over reps calls after one warm-up,
-// launched eagerly on the handle's streams: the same kernels, streams and
-// events as the captured matvec graph, without instantiating a graph per
-// schedule (each instantiate / launch / destroy cycle of a forked graph is
-// one more pass through the runtime's graph launch path, where processes
-// have taken host faults).
-static int time_interior(h2p_hip_handle *h, int reps, double *ms) {
+// Mean time of a matvec behind its gather (interior and leaf outputs, the
+// latter into y) over reps calls after one warm-up, launched eagerly on the
+// handle's streams: the same kernels, streams and events as the captured
+// matvec graph, without instantiating a graph per schedule (each instantiate
+// / launch / destroy cycle of a forked graph is one more pass through the
+// runtime's graph launch path, where processes have taken host faults).  The
+// leaf outputs count for every schedule: where all blocks are one launch they
+// hold the U y1 rows that the others compute in their interior.
+static int time_matvec(h2p_hip_handle *h, int reps, double *y, double *ms) {
     hipStream_t s = h->own_stream;
-    // the leaves' U y1 rows are part of the interior of a split schedule and
-    // of the leaf outputs (here into yt, which these do not read) of the other
-    auto interior = [&] {
+    auto matvec = [&] {
         launch_interior(h, s, nullptr);
-        if (one_launch(h, nullptr)) launch_leaf_out(h, h->d_yt, s, nullptr);
+        launch_leaf_out(h, y, s, nullptr);
     };
-    interior();   // warm-up
+    matvec();   // warm-up
     HIP_TRY(hipGetLastError());
     hipEvent_t e0 = nullptr, e1 = nullptr;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     float t = 0.f;
     int rc = hipEventRecord(e0, s) == hipSuccess ? 0 : fail(H2P_HIP_EDEVICE, "hipEventRecord failed");
-    for (int r = 0; r < reps && !rc; r++) interior();
+    for (int r = 0; r < reps && !rc; r++) matvec();
     if (!rc && (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                 hipEventElapsedTime(&t, e0, e1) != hipSuccess))
-        rc = fail(H2P_HIP_EDEVICE, "timing the matvec interior failed");
+        rc = fail(H2P_HIP_EDEVICE, "timing the matvec schedules failed");
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     *ms = t / reps;
@@ -2094,13 +2094,17 @@ static int autotune_matvec(h2p_hip_handle *h, double *t_default_ms, double *t_tu
         // beside the deep B blocks)
         const int nsch = h->lv_possible ? 4 : 2;
         double ti[4] = {0.0, 0.0, 0.0, 0.0};
-        int bk = 0;
-        for (int k = 0; k < nsch; k++) {
+        int bk = 0, rc = 0;
+        double *y = nullptr;   // outputs of the timed calls
+        if (hipMalloc(&y, sizeof(double) * std::max(h->N, 1)) != hipSuccess)
+            return fail(H2P_HIP_ENOMEM, "hipMalloc of the tuning output failed");
+        for (int k = 0; k < nsch && !rc; k++) {
             set_schedule(h, k);
-            int rc = time_interior(h, 8, &ti[k]);
-            if (rc) return rc;
-            if (ti[k] < ti[bk]) bk = k;
+            rc = time_matvec(h, 8, y, &ti[k]);
+            if (!rc && ti[k] < ti[bk]) bk = k;
         }
+        (void)hipFree(y);
+        if (rc) return rc;
         set_schedule(h, bk);
         code |= ((bk & 1) ? 2 : 0) | ((bk & 2) ? 4 : 0);
     }
