@@ -2041,7 +2041,10 @@ static int autotune_matvec(h2p_hip_handle *h, double *t_default_ms, double *t_tu
         const int b = t.ncol > 0 ? (int)std::floor(std::log2((double)t.ncol)) : -1;
         hist[{a, b}]++;
     }
-    std::string sig = "mv/" + std::to_string(h->kid) + "/" + std::to_string(h->mode) + "/" + std::to_string(h->prec) + ":";
+    // handles with the list of all blocks apart from those without: "in order"
+    // is one launch on the former
+    std::string sig = "mv/" + std::to_string(h->kid) + "/" + std::to_string(h->mode) + "/" + std::to_string(h->prec) +
+                      (h->all.n > 0 ? "/all" : "") + ":";
     for (const auto &e : hist)
         sig += std::to_string(e.first.first) + "," + std::to_string(e.first.second) + "," +
                std::to_string((int)std::floor(std::log2((double)e.second))) + ";";
