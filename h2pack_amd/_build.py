@@ -20,7 +20,7 @@ HOST_SO = os.path.join(PKG, "libh2p_host.so")
 HIP_SO = os.path.join(PKG, "libh2p_hip.so")
 
 HIP_SOURCES = ["h2p_hip.hip"]
-HIP_HEADERS = ["h2p_kernels.h", "h2p_device.h", "h2p_exp2.h", "h2p_mm.h", "h2p_batch.h"]
+HIP_HEADERS = ["h2p_kernels.h", "h2p_device.h", "h2p_exp2.h", "h2p_mm.h", "h2p_batch.h", "h2p_order.h"]
 
 # Packed-FP32 instructions stay disabled: hipcc -O3 would otherwise form
 # v_pk_{add,mul,fma}_f32 from ordinary float code.  MFMA results go to

@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "h2p_hip.h"
+#include "h2p_order.h"
 #include "h2p_kernels.h"
 #include "h2p_mm.h"
 #include "h2p_batch.h"
@@ -1085,11 +1086,12 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
     h->part[3].n = h->split ? nB - nB_deep : 0;
     h->part[1].off = h->split ? nB : h->n_blk;
     h->part[1].n = h->n_blk - h->part[1].off;
+    auto more_work = [](const BlkTask &x, const BlkTask &y) {
+        return (long long)x.nrow * x.ncol > (long long)y.nrow * y.ncol;
+    };
     auto order_part = [&](h2p_hip_handle::BlkPart &P) {
         auto b0 = blk.begin() + P.off, b1 = b0 + P.n;
-        std::stable_sort(b0, b1, [](const BlkTask &x, const BlkTask &y) {
-            return (long long)x.nrow * x.ncol > (long long)y.nrow * y.ncol;
-        });
+        std::stable_sort(b0, b1, more_work);
         P.big = P.n;
         if (tiled)
             P.big = (int)(std::stable_partition(b0, b1, [&](const BlkTask &t) { return !wave_task(t); }) -
@@ -1124,8 +1126,13 @@ static int upload_impl(const h2p_hip_h2pack *g, const h2p_kernel_desc *krnl, int
     if (h->split && h->n_blk > 0 && B_pairs + D_pairs < H2P_ONE_LAUNCH_PAIRS) {
         auto &P = h->all;
         P.off = P.n = h->n_blk;
-        blk.insert(blk.end(), blk.begin(), blk.begin() + h->n_blk);
-        order_part(P);
+        // (the two D parts are one ordered range, cut in two)
+        const auto &B0 = h->part[0], &B1 = h->part[3], &D0 = h->part[1], &D1 = h->part[2];
+        const std::vector<BlkTask> all = merge_parts(
+            blk, {{B0.off, B0.big, B0.n}, {B1.off, B1.big, B1.n}, {D0.off, D0.big + D1.big, D0.n + D1.n}}, more_work,
+            &P.big);
+        blk.insert(blk.end(), all.begin(), all.end());
+        P.units = P.big + (P.n - P.big + 3) / 4;
         h->d_serial = true;
     }
     // ---- active nodes of the downward sweep (y1 "set", src/H2Pack_matvec.c:251-256, :802-838)
