@@ -632,7 +632,7 @@ static void launch_mm(const h2p_hip_handle *h, int kind, const MMTask *tasks, in
     }
 }
 
-// Variant v of one launch: bit 0 picks the task order (the other bit is free).
+// Variant v of one launch: bit 0 picks the task order, bit 1 has no effect.
 static void dispatch_mm(const h2p_hip_handle *h, int kind, const Level &L, const MMPanels &P, hipStream_t s, int v) {
     if (L.n <= 0) return;
     const MMArgs A = mm_args(h, P);

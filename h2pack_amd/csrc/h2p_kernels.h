@@ -206,15 +206,17 @@ __global__ void __launch_bounds__(256) k_reduce_y1(const RedTask *__restrict__ t
 // Sweep kernels.
 //
 // Upward sweep (src/H2Pack_matvec.c:95-177): one workgroup per node and
-// column chunk of its U (256 columns, or 128 / 64 on a level with fewer
+// column chunk of its U (256 columns, or 128 / 64 / 16 on a level with fewer
 // workgroups than CUs, so a node with a large basis spreads over several
-// workgroups); lanes own the chunk's columns (NS strips of 64, only the
-// strips that hold columns), the four waves take contiguous quarters of the
-// rows and load UR = 32 / NS rows x NS strips before their FMAs (32 loads
-// in flight per wave whatever the chunk width, 24 at NS = 3; then 8-row
-// batches, then single rows; rows in order, so each column's sum runs over
-// the rows in order whatever the unrolling and the chunk width); the four
-// wave partials are added in LDS in a fixed order.
+// workgroups).  Chunks of 64 columns and more: lanes own the columns (NS
+// strips of 64, only the strips that hold columns), the four waves take
+// contiguous quarters of the rows and load UR = 32 / NS rows x NS strips
+// before their FMAs (32 loads in flight per wave whatever the chunk width, 24
+// at NS = 3; then 8-row batches, then single rows; rows in order), and the
+// four wave partials are added in LDS in a fixed order: a column's sum has
+// the same bits at each of these widths.  Chunks of 16 columns deal the rows to
+// 16 groups of threads instead (group_dot), another order of the same sum;
+// the width is fixed at upload, so a handle's results do not change.
 // R rows x NS strips loaded, then their FMAs in row order.
 template <int R, int NS>
 __device__ __forceinline__ void fwd2_rows(const double *__restrict__ Ut, int ld, const double *__restrict__ in, int i,
@@ -1070,12 +1072,12 @@ __global__ void __launch_bounds__(256) k_root_block(const double *__restrict__ p
 // lane's tile are evaluated together, their four table reads in flight
 // before the polynomials, and blocks whose values stay normal (H2P_BLK_FAST, 94%
 // of the pairs at N = 1M) add the exponent by an integer operation.  53 instead
-// of 57 VALU operations per tile (Matern: 85 instead of 97); matvec N = 1M
-// Gaussian 13.94 -> 13.60 ms, CG on three Matern matrices of 12-24k points
-// 6.36 -> 5.93 ms per 10 iterations.  A 1024-entry table with a polynomial of one
-// degree less (49 operations) measured slower, 14.5 ms: 8 KB of table to copy
-// per workgroup and more bank conflicts; several units per workgroup, to copy
-// it once, 14.8 ms.
+// of 57 VALU operations per tile (Matern: 85 instead of 97), 65 with staging and
+// reductions (65.5); matvec N = 1M Gaussian 13.63 -> 13.49 ms, CG on three Matern
+// matrices of 12-24k points 6.36 -> 5.93 ms per 10 iterations.  A 1024-entry table
+// with a polynomial of one degree less (49 operations) measured slower, 14.5 ms:
+// 8 KB of table to copy per workgroup and more bank conflicts; several units per
+// workgroup, to copy it once, 14.8 ms.
 #define H2P_JITM_NT 8
 
 // Runs a tile body for the rows that hold points: lane group g's register r

@@ -44,7 +44,7 @@ enum { MM_PX = 0, MM_Y0 = 1, MM_Y1 = 2, MM_PY = 3 };
 enum { MM_A_U = 0, MM_A_UT = 1, MM_A_BD = 2, MM_A_JIT = 3 };
 
 #define H2P_MM_MAXNVP 64
-#define H2P_MM_NVARIANT 4
+#define H2P_MM_NVARIANT 4      // accepted; only bit 0 (the task order) has an effect
 #define H2P_MM_PIECE 32       // rows of a task
 #define H2P_MM_PIECE3 48      // rows of a task with evaluated 3x3 blocks
 

@@ -189,19 +189,20 @@ int h2p_hip_matmul_dev_noalloc(h2p_hip_handle *h, int layout, int n_vec,
 /* Autotuner of the matmul's task orders.  Each matmul phase (upward sweep,
  * coupling, downward sweep, leaf outputs) runs as grouped MFMA launches of
  * tasks in one of two orders: the tasks of a destination on one XCD (even
- * variants, the default) or the longest tasks first (odd variants).  This
- * call times both on the handle's own blocks for panels of n_vec columns and
- * keeps the faster per phase; choices are shared, within the process, by
- * handles whose phase has the same kernel, mode and block-size histogram.
- * Every variant computes bitwise the same result.  Optional outputs: summed
- * phase times of the default variants and of the chosen ones, in
- * milliseconds.
+ * variants, the default) or the longest tasks first (odd variants; 2 and 3
+ * are accepted and launch the same tasks as 0 and 1).  This call times both
+ * on the handle's own blocks for panels of n_vec columns and keeps the faster
+ * per phase; choices are shared, within the process, by handles whose phase
+ * has the same kernel, mode and block-size histogram.  Every variant computes
+ * bitwise the same result.  Optional outputs: summed phase times of the
+ * default variants and of the chosen ones, in milliseconds.
  * n_vec = 0 tunes the matvec instead: its grouped B/D launch has two
  * builds of the same body compiled for different occupancies (JIT: 4 waves
  * per SIMD by default, unconstrained registers as the alternative; AOT:
  * unconstrained by default, 5 (FP64) or 8 (FP32) waves as the
  * alternative), and on JIT handles of the scalar kernels the D blocks run
- * either beside the sweeps on a second stream (default) or in order;
+ * either beside the sweeps on a second stream (the default from 2.5e8 kernel
+ * pairs on) or in order (the default below, with all blocks in one launch);
  * again with identical results.
  * (H2Pack has no counterpart: its products are fixed BLAS / SIMD loops.) */
 #define H2P_HIP_MM_VARIANTS 4
