@@ -357,8 +357,9 @@ def main():
                              "and, with the level split, the shallower levels'), and kernel_ms is their sum "
                              "measured with HIP events in the profiled pass, where they run in order; "
                              "FP64 VALU and FP64 MFMA share the 78.6 TFLOP/s peak (one FP64 pipe: "
-                             "SQ_VALU_MFMA_COEXEC_CYCLES = 0); evaluating a pair issues ~18 pipe slots "
-                             "(2^x 12 FP64/integer operations with its 128-entry LDS table, the squared "
+                             "SQ_VALU_MFMA_COEXEC_CYCLES = 0); evaluating a pair issues ~17 pipe slots "
+                             "(2^x 11 FP64/integer operations with its 128-entry LDS table, 12 and a clamp on "
+                             "blocks with values below 2^-1000, the squared "
                              "distance 4 slots of MFMA, the two products 2), and rocprofv3 counters put the "
                              "pipe ~90% busy (profiles/gaussian_1M_jit_pipe_counters.md)"},
         "cpu_baseline": cpu,

@@ -439,7 +439,7 @@ def run(args):
             tune["tune_s"] = time.perf_counter() - t_t
             dt = _time(mm, K, W, sync)
             Y = Yd.cpu().numpy().T
-            log(f"[bench] rpy {mode}: tile variants {tune['variants']} (phases {tune['default_ms']:.1f} -> "
+            log(f"[bench] rpy {mode}: task orders {tune['variants']} (phases {tune['default_ms']:.1f} -> "
                 f"{tune['tuned_ms']:.1f} ms), matmul {dt_default * 1e3:.1f} -> {dt * 1e3:.1f} ms, "
                 f"identical: {bool(np.array_equal(Y0, Y))}")
             xv = torch.empty(Nk, dtype=torch.float64, device=dev); yv = torch.empty_like(xv)
