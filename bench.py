@@ -361,7 +361,7 @@ def main():
                              "(2^x 11 FP64/integer operations with its 128-entry LDS table, 12 and a clamp on "
                              "blocks with values below 2^-1000, the squared "
                              "distance 4 slots of MFMA, the two products 2), and rocprofv3 counters put the "
-                             "pipe ~90% busy (profiles/gaussian_1M_jit_pipe_counters.md)"},
+                             "pipe ~90% busy (profiles/cases_counters.md)"},
         "cpu_baseline": cpu,
         "serving": serving,
         "rel_err_vs_direct_nbody_1000rows": err_direct,
